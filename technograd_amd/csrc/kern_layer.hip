@@ -14,6 +14,8 @@
 #include "tgm.h"
 
 #include <math.h>
+#include <string.h>
+#include <type_traits>
 
 namespace {
 
@@ -236,13 +238,10 @@ __global__ __launch_bounds__(256) void ew_k(tgk_ew E, int n, int cpr)
 	}
 }
 
-__device__ inline int code_at(const uint8_t *q, int bits, long i)
-{
-	if (bits == 8) return (signed char)q[i];
-	int b = (signed char)q[i >> 1];
-	return (i & 1) ? (b >> 4) : (int)(signed char)(unsigned char)((unsigned)b << 4) >> 4;
-}
-
+// small unquantized products, one thread per output: a thread's operands for
+// eight p are loaded before the first is added, so a load's latency is paid
+// once per eight terms of the chain (512 sequences' mean over 512 steps x 256
+// values, m = 1: 212 to 41 us)
 __global__ void mm_exact_k(tgk_mm d, long total)
 {
 	long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -256,16 +255,16 @@ __global__ void mm_exact_k(tgk_mm d, long total)
 	const float *A = d.a.p + r * d.a.rs + g * d.ag + i * d.ai;
 	const float *B = d.b.p + r * d.b.rs + g * d.bg + (long)j * d.bj;
 	float acc = 0.0f;
-	if (d.quant == 1) {
-		long base = (long)g * d.m * d.k + (long)i * d.k;
-		for (int p = 0; p < d.k; p++) acc += (float)code_at(d.codes, d.bits, base + p) * B[p * d.bp];
-		acc = d.scale[i] * acc;
-	} else if (d.quant == 2) {
-		for (int p = 0; p < d.k; p++) acc += A[p * d.ap] * (float)code_at(d.codes, d.bits, (long)p * d.n + j);
-		acc = d.scale[j] * acc;
-	} else {
-		for (int p = 0; p < d.k; p++) acc += A[p * d.ap] * B[p * d.bp];
+	constexpr int U = 8;
+	int p = 0;
+	for (; p + U <= d.k; p += U) {
+		float x[U], y[U];
+#pragma unroll
+		for (int q = 0; q < U; q++) x[q] = A[(p + q) * d.ap], y[q] = B[(p + q) * d.bp];
+#pragma unroll
+		for (int q = 0; q < U; q++) acc += x[q] * y[q];
 	}
+	for (; p < d.k; p++) acc += A[p * d.ap] * B[p * d.bp];
 	d.o[r * d.ors + g * d.og + i * d.oi + (long)j * d.oj] = acc;
 }
 
@@ -641,11 +640,175 @@ __global__ __launch_bounds__(256) void mm_tile_k(tgk_mm d, int tm, int tn, int n
 	}
 }
 
+// A quantized product in the reference's order: M activation rows (row m =
+// (batch row m / ni, inner row m % ni)) times C channels, o = scale[c] *
+// sum_k code[c][k] x[m][k], products added for k = 0..K-1 from 0.0f with
+// separate multiply and add. It is bound by the VALU (two instructions per
+// term, no fused multiply-add in this order). A block of 16 x 16 threads
+// takes a 16 R x 16 R tile, a thread R x R of its outputs, so R^2 chains hide
+// each other's latency and a value read from LDS serves R of them. Codes
+// become floats once, on the way into LDS; the next chunk's loads are in
+// flight while the current one is multiplied, two LDS buffers leave one
+// barrier per chunk, and within a chunk 16 / R k's of operands are read (16
+// bytes at a time) while the 16 / R before them are used. Terms past K, rows
+// past M and channels past C are 0 code times 0 input: they add +0 to sums
+// that are never -0. 333 rows x 1024 inputs x 1000 int8 channels take 43 us
+// back to back (8 T multiply-adds/s; the products and adds alone issue in
+// 17 us) where one thread per output, a load's latency per term, took 1255.
+struct QExact {
+	int M, C, K, ni;
+	const float *x;
+	long xr, xj, xk;
+	const uint8_t *codes;
+	const float *scale;
+	float *o;
+	long orr, oj, oc;
+	long ck, cc; // code of (channel c, input k) at c * cc + k * ck
+};
+
+template <int R, int BITS>
+__global__ __launch_bounds__(256) void qexact_k(QExact d, int tn)
+{
+	constexpr int KC = 128 / R, TS = 16 * R, NE = TS * KC / 256, ST = KC + 4; // NE: elements per thread, chunk and operand
+	constexpr int G = 16 / R, NG = KC / G;                                  // k's per group of LDS reads, groups per chunk
+	__shared__ __align__(16) float Xs[2][TS][ST], Ws[2][TS][ST];            // rows 4 banks apart: 16 lanes' 16-byte reads meet no bank twice
+	const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+	const int tm0 = (int)(blockIdx.x / (unsigned)tn) * TS, c0 = (int)(blockIdx.x % (unsigned)tn) * TS;
+	// element e = tid + 256 q of a chunk: along whichever of the two is unit stride in memory. Every load is made, at
+	// row, channel and input 0 where there is none, and the value dropped after: loads under a condition would wait
+	// for each other
+	const bool xp = d.xk == 1, wp = d.ck == 1;
+	float rx[NE];
+	int rw[NE];
+	const float *xa[NE]; // the element in x, and its code's index, in the chunk to be loaded next
+	long wa[NE];
+	int xk[NE], wk[NE]; // its input in the chunk (K: no such row or channel)
+	for (int q = 0; q < NE; q++) {
+		const int e = tid + q * 256, m = tm0 + (xp ? e / KC : e % TS), c = c0 + (wp ? e / KC : e % TS);
+		xk[q] = xp ? e % KC : e / TS, wk[q] = wp ? e % KC : e / TS;
+		xa[q] = d.x + (m < d.M ? (long)(m / d.ni) * d.xr + (long)(m % d.ni) * d.xj : 0) + (long)xk[q] * d.xk;
+		wa[q] = (c < d.C ? (long)c * d.cc : 0) + (long)wk[q] * d.ck;
+		if (m >= d.M) xk[q] = d.K;
+		if (c >= d.C) wk[q] = d.K;
+	}
+	const long xstep = KC * d.xk, wstep = KC * d.ck;
+	auto fetch = [&](int p0) {
+#pragma unroll
+		for (int q = 0; q < NE; q++) {
+			rx[q] = *(p0 + xk[q] < d.K ? xa[q] : d.x);
+			xa[q] += xstep;
+		}
+#pragma unroll
+		for (int q = 0; q < NE; q++) {
+			const long i = p0 + wk[q] < d.K ? wa[q] : 0;
+			rw[q] = BITS == 8 ? (int)(int8_t)d.codes[i] : (int)(int8_t)(uint8_t)(d.codes[i >> 1] << (i & 1 ? 0 : 4)) >> 4;
+			wa[q] += wstep;
+		}
+#pragma unroll
+		for (int q = 0; q < NE; q++) {
+			rx[q] = p0 + xk[q] < d.K ? rx[q] : 0.0f;
+			rw[q] = p0 + wk[q] < d.K ? rw[q] : 0;
+		}
+	};
+	auto stash = [&](int b) {
+#pragma unroll
+		for (int q = 0; q < NE; q++) {
+			const int e = tid + q * 256;
+			if (xp) Xs[b][e / KC][e % KC] = rx[q];
+			else Xs[b][e % TS][e / TS] = rx[q];
+			if (wp) Ws[b][e / KC][e % KC] = (float)rw[q];
+			else Ws[b][e % TS][e / TS] = (float)rw[q];
+		}
+	};
+	float acc[R][R];
+	for (int u = 0; u < R; u++)
+		for (int v = 0; v < R; v++) acc[u][v] = 0.0f;
+	fetch(0);
+	stash(0);
+	__syncthreads();
+	for (int p0 = 0, b = 0; p0 < d.K; p0 += KC, b ^= 1) {
+		const bool more = p0 + KC < d.K;
+		if (more) fetch(p0 + KC);
+		float4 x[2][R][G / 4], w[2][R][G / 4]; // two groups in turn
+		auto read = [&](int s, int g) {
+#pragma unroll
+			for (int u = 0; u < R; u++)
+#pragma unroll
+				for (int i = 0; i < G / 4; i++) {
+					x[s][u][i] = *(const float4 *)&Xs[b][u * 16 + ty][g * G + 4 * i];
+					w[s][u][i] = *(const float4 *)&Ws[b][u * 16 + tx][g * G + 4 * i];
+				}
+		};
+		auto terms = [&](int s) {
+#pragma unroll
+			for (int i = 0; i < G / 4; i++) {
+#define QX_TERM(K) 	_Pragma("unroll") for (int u = 0; u < R; u++) _Pragma("unroll") for (int v = 0; v < R; v++) acc[u][v] = acc[u][v] + w[s][v][i].K * x[s][u][i].K;
+				QX_TERM(x) QX_TERM(y) QX_TERM(z) QX_TERM(w)
+#undef QX_TERM
+			}
+		};
+		read(0, 0);
+		const int ng = d.K - p0 >= KC ? NG : (d.K - p0 + G - 1) / G; // groups with a term of the product
+#pragma unroll
+		for (int g = 0; g < NG; g += 2) {
+			if (g >= ng) break;
+			read(1, g + 1);
+			terms(0);
+			if (g + 2 < NG) read(0, g + 2);
+			if (g + 1 < ng) terms(1);
+		}
+		if (more) stash(b ^ 1); // the other buffer: its last readers are past the barrier before this chunk
+		__syncthreads();
+	}
+	for (int u = 0; u < R; u++) {
+		const int m = tm0 + u * 16 + ty;
+		if (m >= d.M) break;
+		float *o = d.o + (long)(m / d.ni) * d.orr + (long)(m % d.ni) * d.oj;
+		for (int v = 0; v < R; v++) {
+			const int c = c0 + v * 16 + tx;
+			if (c < d.C) o[(long)c * d.oc] = d.scale[c] * acc[u][v];
+		}
+	}
+}
+
+// the quantized products of tgk_matmul_exact (g == 1)
+static void launch_qexact(hipStream_t s, const tgk_mm *d, int rows)
+{
+	QExact e;
+	memset(&e, 0, sizeof e);
+	const bool left = d->quant == 1; // codes on the left: o = diag(scale) Q @ b
+	e.K = d->k, e.codes = d->codes, e.scale = d->scale, e.o = d->o, e.orr = d->ors;
+	e.C = left ? d->m : d->n, e.ni = left ? d->n : d->m;
+	e.x = left ? d->b.p : d->a.p;
+	e.xr = left ? d->b.rs : d->a.rs, e.xj = left ? d->bj : d->ai, e.xk = left ? d->bp : d->ap;
+	e.oc = left ? d->oi : d->oj, e.oj = left ? d->oj : d->oi;
+	e.cc = left ? d->k : 1, e.ck = left ? 1 : d->n;
+	const long M = (long)rows * e.ni;
+	e.M = (int)M;
+	auto tiles = [&](int ts) { return ((M + ts - 1) / ts) * ((e.C + ts - 1) / ts); };
+	// A round of 256 blocks (one a compute unit) of 1024 inputs takes about 17, 37 and 97 us for R = 1, 2 and 4; a
+	// unit's second block runs beside the first at R = 1 and 2 (22 and 49 us). So R = 2 from 256 of its tiles
+	// (333 rows x 1000 channels: 49 us against 57 at R = 1; 128 rows: 39 against 22), and R = 4, which does the
+	// most per LDS read, once its tiles fill the chip twice (4096 rows: 286 us against 390).
+	auto run = [&](auto bits) {
+		constexpr int B = decltype(bits)::value;
+		if (tiles(64) >= 512) qexact_k<4, B><<<(unsigned)tiles(64), 256, 0, s>>>(e, (e.C + 63) / 64);
+		else if (tiles(32) >= 256) qexact_k<2, B><<<(unsigned)tiles(32), 256, 0, s>>>(e, (e.C + 31) / 32);
+		else qexact_k<1, B><<<(unsigned)tiles(16), 256, 0, s>>>(e, (e.C + 15) / 16);
+	};
+	if (d->bits == 8) run(std::integral_constant<int, 8>{});
+	else run(std::integral_constant<int, 4>{});
+}
+
 void tgk_matmul_exact(hipStream_t s, const tgk_mm *d, int rows)
 {
 	long total = (long)rows * d->g * d->m * d->n;
 	if (total <= 0) return;
-	if (d->quant == 0 && (long)d->m * d->n >= 64 * 64 && d->k >= 16) {
+	if (d->quant) {
+		launch_qexact(s, d, rows);
+		return;
+	}
+	if ((long)d->m * d->n >= 64 * 64 && d->k >= 16) {
 		const long rg = (long)rows * d->g;
 		if (d->causal == 1 && d->m == d->n) { // 64 x 64 tiles on or below the diagonal
 			const int nt = (d->m + 63) / 64, ntri = nt * (nt + 1) / 2;
