@@ -790,49 +790,74 @@ __global__ __launch_bounds__(256) void silu_mul_k(const float *gu, long gus, flo
 	}
 }
 
-// A prompt chunk's causal softmax of one head's scores, line (sequence, t)
-// of sc = q_t . k_u for u <= t (the products above the diagonal are not
-// computed). The graph's operations on the valid part: x_u = s_u * scale + 0
-// (the mask's 0), the row op's max rule, expf(x_u - max), the sum in key
-// order, e_u / sum. Above the diagonal the graph adds -1e9: for finite scores
-// that entry never wins the max and its expf is exactly 0, which leaves the
-// sum unchanged and gives p_u = 0, written here directly. lpb lines per block
-// (a power of two >= 4) staged in LDS, stride T0 + 4 floats (16-byte aligned).
-__global__ __launch_bounds__(256) void causal_softmax_k(float *sc, int T0, long nlines, float scale, int lpb, int stride)
+// A prompt chunk's causal softmax, line (sequence, head, t) of sc = q_t . k_u
+// for u <= t (the products above the diagonal are not computed). The graph's
+// operations on the valid part: x_u = s_u * scale + 0 (the mask's 0), the row
+// op's max rule, expf(x_u - max), the sum in key order, e_u / sum. Above the
+// diagonal the graph adds -1e9: for finite scores that entry never wins the
+// max and its expf is exactly 0, which leaves the sum unchanged and gives
+// p_u = 0, written here directly, up to the end of the line's tile of ztile
+// positions. lpb lines per block (a power of two >= 4) staged in LDS, stride
+// T0 + 4 floats (16-byte aligned); 256 / lpb lanes of one wave take a line, V
+// consecutive elements each, so its max and its exponentials need no barrier,
+// and only the ordered sums, one thread per line, side by side in one wave,
+// do. A line's sum is one chain of adds: eight lines a block leave room for
+// eight blocks a compute unit, whose chains overlap (16 x 16 lines of 512
+// positions: 111 us; 193 when the block's lanes went through its lines one after
+// another, 279 so at 32 lines a block, and 448 a head at a time).
+template <int V>
+__global__ __launch_bounds__(256) void causal_softmax_k(float *sc, int T0, long nlines, float scale, int ztile, int lpb, int stride)
 {
 	extern __shared__ float4 sh4[];
-	float *z = (float *)sh4, *lv = z + lpb * stride; // lv: per line max, then sum
+	float *z = (float *)sh4, *lv = z + lpb * stride; // lv: per line its sum
 	const long L0 = (long)blockIdx.x * lpb;
-	const int tid = threadIdx.x, t0 = (int)(L0 % T0);
-	const int nl = nlines - L0 < lpb ? (int)(nlines - L0) : lpb; // lines of this block
-	auto pos = [&](int ll) { return (t0 + ll) % T0; };          // line ll's position t
-	for (int ll = 0; ll < nl; ll++) {
-		const int t = pos(ll);
-		const float *src = sc + (L0 + ll) * T0;
-		for (int u = tid; u <= t; u += 256) z[ll * stride + u] = src[u] * scale + 0.0f;
+	const int tid = threadIdx.x, tpl = 256 / lpb, l = tid / tpl, sub = tid - l * tpl;
+	const long L = L0 + l;
+	const int t = L < nlines ? (int)((unsigned)L % (unsigned)T0) : -1; // the line's position (none: no elements)
+	float *y = z + l * stride, *line = sc + L * T0, m = -INFINITY, y0 = 0.0f;
+	constexpr int U = 4;
+	const int step = tpl * V;
+	for (int u0 = sub * V; u0 <= t; u0 += U * step) { // U loads in flight
+		float x[U][V];
+#pragma unroll
+		for (int q = 0; q < U; q++) {
+			const int u = u0 + q * step <= t ? u0 + q * step : u0;
+			if constexpr (V == 4) {
+				const float4 s4 = *(const float4 *)(line + u);
+				x[q][0] = s4.x, x[q][1] = s4.y, x[q][2] = s4.z, x[q][3] = s4.w;
+			} else
+				x[q][0] = line[u];
+		}
+#pragma unroll
+		for (int q = 0; q < U; q++) {
+			const int u = u0 + q * step;
+			if (u > t) break;
+#pragma unroll
+			for (int i = 0; i < V; i++) {
+				x[q][i] = x[q][i] * scale + 0.0f;
+				y[u + i] = x[q][i];
+				if (u + i == 0) y0 = x[q][i];
+				else if (u + i <= t) m = fmaxf(m, x[q][i]);
+			}
+		}
 	}
+	for (int w = tpl / 2; w > 0; w >>= 1) m = fmaxf(m, __shfl_xor(m, w));
+	y0 = __shfl(y0, (tid & 63) - sub); // the lane that holds the line's first element
+	m = isnan(y0) ? y0 : fmaxf(y0, m);
+	for (int u = sub * V; u <= t; u += step)
+#pragma unroll
+		for (int i = 0; i < V; i++) y[u + i] = expf(y[u + i] - m);
 	__syncthreads();
-	{ // max: 256 / lpb consecutive lanes of one wave per line
-		const int tpl = 256 / lpb, l = tid / tpl, sub = tid - l * tpl;
-		const int t = l < nl ? pos(l) : 0;
-		const float *y = z + l * stride;
-		float m = -INFINITY;
-		for (int u = 1 + sub; u <= t; u += tpl) m = fmaxf(m, y[u]);
-		for (int w = tpl / 2; w > 0; w >>= 1) m = fmaxf(m, __shfl_xor(m, w));
-		if (sub == 0) lv[l] = isnan(y[0]) ? y[0] : fmaxf(y[0], m);
-	}
+	if (tid < lpb && L0 + tid < nlines) lv[tid] = tg_ordered_sum_pp<6>(z + tid * stride, (int)((unsigned)(L0 + tid) % (unsigned)T0) + 1);
 	__syncthreads();
-	for (int ll = 0; ll < nl; ll++) {
-		const int t = pos(ll);
-		for (int u = tid; u <= t; u += 256) z[ll * stride + u] = expf(z[ll * stride + u] - lv[ll]);
-	}
-	__syncthreads();
-	if (tid < nl) lv[tid] = tg_ordered_sum_pp<6>(z + tid * stride, pos(tid) + 1);
-	__syncthreads();
-	for (int ll = 0; ll < nl; ll++) {
-		const int t = pos(ll);
-		float *dst = sc + (L0 + ll) * T0;
-		for (int u = tid; u < T0; u += 256) dst[u] = u <= t ? z[ll * stride + u] / lv[ll] : 0.0f;
+	const float sum = lv[l];
+	const int zend = t < 0 ? 0 : min(T0, (t / ztile + 1) * ztile);
+	for (int u = sub * V; u < zend; u += step) {
+		float p[V];
+#pragma unroll
+		for (int i = 0; i < V; i++) p[i] = u + i <= t ? y[u + i] / sum : 0.0f;
+		if constexpr (V == 4) *(float4 *)(line + u) = make_float4(p[0], p[1], p[2], p[3]);
+		else line[u] = p[0];
 	}
 }
 
@@ -991,13 +1016,17 @@ bool tgk_dec_silu(hipStream_t s, const tgk_dec_silu_args *a)
 	return true;
 }
 
-void tgk_dec_causal_softmax(hipStream_t s, float *sc, int T0, long nlines, float scale)
+void tgk_dec_causal_softmax(hipStream_t s, float *sc, int T0, long nlines, float scale, int ztile)
 {
 	if (nlines <= 0 || T0 <= 0) return;
 	const int stride = (T0 + 3) / 4 * 4 + 4;
-	int lpb = 64; // a power of two >= 4: lines per block
+	int lpb = 8; // a power of two >= 4: lines per block, more of short lines so that every lane has elements
+	while (lpb < 64 && lpb * T0 < 1024) lpb <<= 1;
 	while (lpb > 4 && (long)lpb * stride * 4 + lpb * 4 > 65536) lpb >>= 1;
-	causal_softmax_k<<<(unsigned)((nlines + lpb - 1) / lpb), 256, (size_t)lpb * stride * 4 + lpb * 4, s>>>(sc, T0, nlines, scale, lpb, stride);
+	const unsigned grid = (unsigned)((nlines + lpb - 1) / lpb);
+	const size_t lds = (size_t)lpb * stride * 4 + lpb * 4;
+	if (T0 % 4 == 0 && ((size_t)sc & 15) == 0) causal_softmax_k<4><<<grid, 256, lds, s>>>(sc, T0, nlines, scale, ztile ? ztile : T0, lpb, stride);
+	else causal_softmax_k<1><<<grid, 256, lds, s>>>(sc, T0, nlines, scale, ztile ? ztile : T0, lpb, stride);
 }
 
 size_t tgk_dec_wo_lds(int rows, int HD)

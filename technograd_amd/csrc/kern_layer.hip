@@ -253,7 +253,7 @@ __global__ void mm_exact_k(tgk_mm d, long total)
 	int g = (int)(u % d.g);
 	long r = u / d.g;
 	const float *A = d.a.p + r * d.a.rs + g * d.ag + i * d.ai;
-	const float *B = d.b.p + r * d.b.rs + g * d.bg + (long)j * d.bj;
+	const float *B = d.b.p + r * d.b.rs + (d.gb > 1 ? g / d.gb : g) * d.bg + (long)j * d.bj;
 	float acc = 0.0f;
 	constexpr int U = 8;
 	int p = 0;
@@ -523,81 +523,138 @@ void tgk_ew_run(hipStream_t s, const tgk_ew *e, int n, int rows)
 	}
 }
 
-// f32 products (quant 0) in tiles: a block computes a TS x TS tile of one
-// (batch row, group) product, each of its 16 x 16 threads a TS/16 x TS/16
-// block of it. A and B pass through LDS 16 values of p at a time, and every
+// f32 products in tiles: a block of 16 x 16 threads computes a 64 x 64 tile
+// of one (batch row, group) product, a thread 4 x 4 of its outputs. Every
 // output adds its products in order p = 0..kend-1 from 0.0f with separate
 // multiply and add, exactly as mm_exact_k does, so the results are
-// bit-identical to it. Tile rows, columns and p values past m, n and k read
-// as zeros; the p loop stops at kend and nothing past m or n is stored.
-template <int TS>
-__device__ inline void mm_tile(const tgk_mm &d, const float *A, const float *B, float *O, int i0, int j0, int kend, float (*As)[TS + 4],
-			       float (*Bs)[TS + 4])
+// bit-identical to it; that order makes two VALU instructions per product the
+// bound. A and B pass through LDS 32 values of p at a time: the next chunk's
+// loads are in flight while the current one is multiplied, two LDS buffers
+// leave one barrier per chunk, and four p's of operands (eight 16-byte reads
+// for 128 VALU instructions) are read while the four before them are used. An
+// operand contiguous along p lies in LDS as [row][p], any other as [p][row],
+// so both are filled and read 16 bytes at a time. Tile rows, columns and p
+// values past m, n and k read as zeros in both operands (they add +0 to sums
+// that are never -0); nothing past m or n is stored. 256 causal products of
+// 512 x 512 x 128 (16 heads of 16 sequences) take 240 us, 20 T multiply-adds/s:
+// the VALU's issue rate. The former tiles (16 p's a chunk, operands read four
+// at a time as they were used) took about 60 us for a head's 16, launched
+// alone (960 us for the 256; two and a quarter blocks a compute unit), and
+// 128 x 128 of them 66-72 % of the issue rate on the full square.
+constexpr int MT = TGK_MM_TILE, MKC = 32;
+
+// One operand of a tile, element (row, p) at base + row rs + p ps: the
+// thread's two quads of each chunk. KMAJ: contiguous along p, LDS [MT][MKC +
+// 4], else LDS [MKC][MT + 4]. VEC: every quad is 16-byte aligned and wholly
+// inside or outside the operand. A quad outside is loaded from the base and
+// dropped: loads under a condition would wait for each other.
+template <bool KMAJ, bool VEC>
+struct MmOpd {
+	static constexpr int NQ = (KMAJ ? MKC : MT) / 4, LD = 4 * NQ + 4, FLOATS = (KMAJ ? MT : MKC) * LD;
+	const float *base, *a[2];
+	float4 v[2];
+	long step, qs; // one chunk on; from a quad's element to its next
+	int row[2], p[2], rows, k;
+	__device__ inline void init(const float *base_, long rs, long ps, int row0, int rows_, int k_)
+	{
+		base = base_, rows = rows_, k = k_, step = MKC * ps, qs = KMAJ ? ps : rs;
+#pragma unroll
+		for (int q = 0; q < 2; q++) {
+			const int e = threadIdx.x + q * 256, l = e / NQ, c = 4 * (e % NQ);
+			row[q] = row0 + (KMAJ ? l : c), p[q] = KMAJ ? c : l;
+			a[q] = base + (long)row[q] * rs + (long)p[q] * ps;
+		}
+	}
+	__device__ inline void fetch() // the next chunk's quads
+	{
+#pragma unroll
+		for (int q = 0; q < 2; q++) {
+			if constexpr (VEC) {
+				v[q] = *(const float4 *)(row[q] < rows && p[q] < k ? a[q] : base);
+			} else {
+				auto at = [&](int i) { return row[q] + (KMAJ ? 0 : i) < rows && p[q] + (KMAJ ? i : 0) < k ? a[q] + i * qs : base; };
+				v[q] = make_float4(*at(0), *at(1), *at(2), *at(3));
+			}
+		}
+#pragma unroll
+		for (int q = 0; q < 2; q++) {
+			auto in = [&](int i) { return row[q] + (KMAJ || VEC ? 0 : i) < rows && p[q] + (KMAJ && !VEC ? i : 0) < k; };
+			v[q] = make_float4(in(0) ? v[q].x : 0.0f, in(1) ? v[q].y : 0.0f, in(2) ? v[q].z : 0.0f, in(3) ? v[q].w : 0.0f);
+			a[q] += step, p[q] += MKC;
+		}
+	}
+	__device__ inline void stash(float *z) const
+	{
+#pragma unroll
+		for (int q = 0; q < 2; q++) {
+			const int e = threadIdx.x + q * 256;
+			*(float4 *)(z + (e / NQ) * LD + 4 * (e % NQ)) = v[q];
+		}
+	}
+	// the tile row of a thread's u-th output on this side (t = its index of 16)
+	static __device__ inline int at(int t, int u) { return KMAJ ? u * 16 + t : t * 4 + u; }
+	// its values of p = 4 g .. 4 g + 3: KMAJ w[u] = row u's four p's, else w[i] = p i's four rows
+	static __device__ inline void read(const float *z, int t, int g, float4 (&w)[4])
+	{
+#pragma unroll
+		for (int u = 0; u < 4; u++) w[u] = *(const float4 *)(KMAJ ? z + at(t, u) * LD + 4 * g : z + (4 * g + u) * LD + 4 * t);
+	}
+	static __device__ inline float get(const float4 (&w)[4], int u, int i) // row u, p i
+	{
+		const float4 x = KMAJ ? w[u] : w[i];
+		const int j = KMAJ ? i : u;
+		return j == 0 ? x.x : j == 1 ? x.y : j == 2 ? x.z : x.w;
+	}
+};
+
+template <class OA, class OB>
+__device__ inline void mm_tile(const tgk_mm &d, const float *A, const float *B, float *O, int i0, int j0, int kend, float *As, float *Bs)
 {
-	constexpr int KC = 16, R = TS / 16, NE = TS * KC / 256; // tile elements per thread and chunk
 	const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-	float acc[R][R];
-	for (int u = 0; u < R; u++)
-		for (int v = 0; v < R; v++) acc[u][v] = 0.0f;
-	// chunk p0's A and B elements of this thread into registers (the next
-	// chunk's loads are in flight while the current one is multiplied)
-	float ra[NE], rb[NE];
-	auto fetch = [&](int p0) {
-		for (int q = 0; q < NE; q++) { // A, coalesced along whichever of i, p is unit stride
-			const int e = threadIdx.x + q * 256;
-			int i, p;
-			if (d.ap == 1) i = e / KC, p = e % KC;
-			else p = e / TS, i = e % TS;
-			const bool in = i0 + i < d.m && p0 + p < d.k;
-			const float x = A[in ? (long)(i0 + i) * d.ai + (long)(p0 + p) * d.ap : 0];
-			ra[q] = in ? x : 0.0f;
-		}
-		for (int q = 0; q < NE; q++) { // B
-			const int e = threadIdx.x + q * 256;
-			int j, p;
-			if (d.bj == 1 || d.bp != 1) p = e / TS, j = e % TS;
-			else j = e / KC, p = e % KC;
-			const bool in = j0 + j < d.n && p0 + p < d.k;
-			const float x = B[in ? (long)(p0 + p) * d.bp + (long)(j0 + j) * d.bj : 0];
-			rb[q] = in ? x : 0.0f;
-		}
-	};
-	auto stash = [&]() {
-		for (int q = 0; q < NE; q++) {
-			const int e = threadIdx.x + q * 256;
-			if (d.ap == 1) As[e % KC][e / KC] = ra[q];
-			else As[e / TS][e % TS] = ra[q];
-			if (d.bj == 1 || d.bp != 1) Bs[e / TS][e % TS] = rb[q];
-			else Bs[e % KC][e / KC] = rb[q];
-		}
-	};
-	if (kend > 0) {
-		fetch(0);
-		stash();
-	}
+	OA oa;
+	OB ob;
+	oa.init(A, d.ai, d.ap, i0, d.m, d.k);
+	ob.init(B, d.bj, d.bp, j0, d.n, d.k);
+	float acc[4][4];
+#pragma unroll
+	for (int u = 0; u < 4; u++)
+#pragma unroll
+		for (int v = 0; v < 4; v++) acc[u][v] = 0.0f;
+	oa.fetch(), ob.fetch();
+	oa.stash(As), ob.stash(Bs);
 	__syncthreads();
-	for (int p0 = 0; p0 < kend; p0 += KC) {
-		const bool more = p0 + KC < kend;
-		if (more) fetch(p0 + KC);
-		const int kk = kend - p0 < KC ? kend - p0 : KC;
-		for (int p = 0; p < kk; p++) {
-			float a[R], b[R];
-			for (int u = 0; u < R; u++) a[u] = As[p][ty * R + u];
-			for (int v = 0; v < R; v++) b[v] = Bs[p][tx * R + v];
-			for (int u = 0; u < R; u++)
-				for (int v = 0; v < R; v++) acc[u][v] = acc[u][v] + a[u] * b[v];
+	for (int p0 = 0, b = 0; p0 < kend; p0 += MKC, b ^= 1) {
+		const bool more = p0 + MKC < kend;
+		if (more) oa.fetch(), ob.fetch();
+		const float *za = As + b * OA::FLOATS, *zb = Bs + b * OB::FLOATS;
+		float4 x0[4], w0[4], x1[4], w1[4]; // two groups of four p's in turn
+		auto terms = [&](const float4 (&x)[4], const float4 (&w)[4]) {
+#pragma unroll
+			for (int i = 0; i < 4; i++)
+#pragma unroll
+				for (int u = 0; u < 4; u++)
+#pragma unroll
+					for (int v = 0; v < 4; v++) acc[u][v] = acc[u][v] + OA::get(x, u, i) * OB::get(w, v, i);
+		};
+		OA::read(za, ty, 0, x0), OB::read(zb, tx, 0, w0);
+#pragma unroll 1 // (unrolled, every read moves to the top of the chunk and spills)
+		for (int g = 0; g < MKC / 4; g += 2) {
+			OA::read(za, ty, g + 1, x1), OB::read(zb, tx, g + 1, w1);
+			terms(x0, w0);
+			const int n = (g + 2) % (MKC / 4); // (the last read is not used)
+			OA::read(za, ty, n, x0), OB::read(zb, tx, n, w0);
+			terms(x1, w1);
 		}
+		if (more) oa.stash(As + (b ^ 1) * OA::FLOATS), ob.stash(Bs + (b ^ 1) * OB::FLOATS); // (its last readers are a barrier behind)
 		__syncthreads();
-		if (more) {
-			stash();
-			__syncthreads();
-		}
 	}
-	for (int u = 0; u < R; u++) {
-		const int i = i0 + ty * R + u;
-		if (i >= d.m) break;
-		for (int v = 0; v < R; v++) {
-			const int j = j0 + tx * R + v;
+#pragma unroll
+	for (int u = 0; u < 4; u++) {
+		const int i = i0 + OA::at(ty, u);
+		if (i >= d.m) continue;
+#pragma unroll
+		for (int v = 0; v < 4; v++) {
+			const int j = j0 + OB::at(tx, v);
 			if (j < d.n) O[(long)i * d.oi + (long)j * d.oj] = acc[u][v];
 		}
 	}
@@ -608,36 +665,60 @@ __device__ inline void mm_tile(const tgk_mm &d, const float *A, const float *B, 
 // (tn counts them, ti >= tj, all of equal work); mode 2 gives a block the row
 // tiles p and tm - 1 - p of one column tile (tm counts the pairs), whose sums
 // run to the end of each tile's rows, so every block has the same work.
-template <int TS>
-__global__ __launch_bounds__(256) void mm_tile_k(tgk_mm d, int tm, int tn, int nt, int mode)
+template <bool AK, bool BK, bool VEC>
+__global__ __launch_bounds__(256, 3) void mm_tile_k(tgk_mm d, int tm, int tn, int nt, int mode)
 {
-	__shared__ float As[16][TS + 4]; // As[p][i]
-	__shared__ float Bs[16][TS + 4]; // Bs[p][j]
+	using OA = MmOpd<AK, VEC>;
+	using OB = MmOpd<BK, VEC>;
+	__shared__ __align__(16) float As[2 * OA::FLOATS], Bs[2 * OB::FLOATS];
 	const int tiles = tm * tn;
 	const long rg = blockIdx.x / tiles;
 	const int t = (int)(blockIdx.x - rg * tiles);
 	const long r = rg / d.g;
 	const int g = (int)(rg - r * d.g);
-	const float *A = d.a.p + r * d.a.rs + g * d.ag, *B = d.b.p + r * d.b.rs + g * d.bg;
+	const float *A = d.a.p + r * d.a.rs + g * d.ag, *B = d.b.p + r * d.b.rs + (d.gb > 1 ? g / d.gb : g) * d.bg;
 	float *O = d.o + r * d.ors + g * d.og;
+	int ti = t / tn, tj = t - ti * tn, other = -1;
 	if (mode == 1) { // lower-triangle tile t: ti (ti + 1) / 2 <= t < (ti + 1) (ti + 2) / 2
-		int ti = (int)((sqrtf(8.0f * t + 1.0f) - 1.0f) * 0.5f);
+		ti = (int)((sqrtf(8.0f * t + 1.0f) - 1.0f) * 0.5f);
 		while (ti * (ti + 1) / 2 > t) ti--;
 		while ((ti + 1) * (ti + 2) / 2 <= t) ti++;
-		const int tj = t - ti * (ti + 1) / 2;
-		mm_tile<TS>(d, A, B, O, ti * TS, tj * TS, d.k, As, Bs);
-	} else if (mode == 2) {
-		const int pr = t / tn, tj = t - pr * tn;
-		for (int h = 0; h < 2; h++) {
-			const int ti = h == 0 ? pr : nt - 1 - pr;
-			if (h == 1 && ti == pr) break; // the middle tile of an odd count
-			const int i0 = ti * TS, kend = i0 + TS < d.k ? i0 + TS : d.k;
-			mm_tile<TS>(d, A, B, O, i0, tj * TS, kend, As, Bs);
-		}
-	} else {
-		const int ti = t / tn, tj = t - ti * tn;
-		mm_tile<TS>(d, A, B, O, ti * TS, tj * TS, d.k, As, Bs);
+		tj = t - ti * (ti + 1) / 2;
+	} else if (mode == 2 && nt - 1 - ti != ti) { // (an odd count's middle tile stands alone)
+		other = nt - 1 - ti;
 	}
+	for (;; ti = other, other = -1) {
+		const int i0 = ti * MT, kend = mode == 2 && i0 + MT < d.k ? i0 + MT : d.k;
+		mm_tile<OA, OB>(d, A, B, O, i0, tj * MT, kend, As, Bs);
+		if (other < 0) break;
+	}
+}
+
+bool tgk_mm_tiled(const tgk_mm *d) { return !d->quant && (long)d->m * d->n >= 64 * 64 && d->k >= 16; }
+
+static void launch_mm_tile(hipStream_t s, const tgk_mm *d, int rows)
+{
+	const long rg = (long)rows * d->g;
+	const int nt = (d->m + MT - 1) / MT, sn = (d->n + MT - 1) / MT;
+	int tm = nt, tn = sn, mode = 0;
+	if (d->causal == 1 && d->m == d->n) tm = 1, tn = nt * (nt + 1) / 2, mode = 1; // tiles on or below the diagonal
+	else if (d->causal == 2) tm = (nt + 1) / 2, mode = 2;                        // pairs of row tiles
+	const bool ak = d->ap == 1, bk = d->bp == 1 && d->bj != 1;
+	// 16-byte loads: aligned bases and row strides, and a contiguous extent of whole quads
+	auto vec = [](const float *p, long rs, long gs, bool kmaj, long row, long ps, int nrow, int k) {
+		return ((size_t)p & 15) == 0 && rs % 4 == 0 && gs % 4 == 0 && (kmaj ? row % 4 == 0 && k % 4 == 0 : row == 1 && ps % 4 == 0 && nrow % 4 == 0);
+	};
+	const bool v = vec(d->a.p, d->a.rs, d->g > 1 ? d->ag : 0, ak, d->ai, d->ap, d->m, d->k) &&
+		       vec(d->b.p, d->b.rs, d->g > 1 ? d->bg : 0, bk, d->bj, d->bp, d->n, d->k);
+	const unsigned grid = (unsigned)(rg * tm * tn);
+	auto run = [&](auto AK, auto BK) {
+		if (v) mm_tile_k<AK.value, BK.value, true><<<grid, 256, 0, s>>>(*d, tm, tn, nt, mode);
+		else mm_tile_k<AK.value, BK.value, false><<<grid, 256, 0, s>>>(*d, tm, tn, nt, mode);
+	};
+	if (ak && bk) run(std::true_type{}, std::true_type{});
+	else if (ak) run(std::true_type{}, std::false_type{});
+	else if (bk) run(std::false_type{}, std::true_type{});
+	else run(std::false_type{}, std::false_type{});
 }
 
 // A quantized product in the reference's order: M activation rows (row m =
@@ -808,25 +889,8 @@ void tgk_matmul_exact(hipStream_t s, const tgk_mm *d, int rows)
 		launch_qexact(s, d, rows);
 		return;
 	}
-	if ((long)d->m * d->n >= 64 * 64 && d->k >= 16) {
-		const long rg = (long)rows * d->g;
-		if (d->causal == 1 && d->m == d->n) { // 64 x 64 tiles on or below the diagonal
-			const int nt = (d->m + 63) / 64, ntri = nt * (nt + 1) / 2;
-			mm_tile_k<64><<<(unsigned)(rg * ntri), 256, 0, s>>>(*d, 1, ntri, nt, 1);
-			return;
-		}
-		if (d->causal == 2) { // pairs of 64-row tiles
-			const int nt = (d->m + 63) / 64, sn = (d->n + 63) / 64;
-			mm_tile_k<64><<<(unsigned)(rg * ((nt + 1) / 2) * sn), 256, 0, s>>>(*d, (nt + 1) / 2, sn, nt, 2);
-			return;
-		}
-		const int tm = (d->m + 127) / 128, tn = (d->n + 127) / 128;
-		if (rg * tm * tn >= 1024) { // enough 128 x 128 tiles to fill the chip
-			mm_tile_k<128><<<(unsigned)(rg * tm * tn), 256, 0, s>>>(*d, tm, tn, tm, 0);
-		} else {
-			const int sm = (d->m + 63) / 64, sn = (d->n + 63) / 64;
-			mm_tile_k<64><<<(unsigned)(rg * sm * sn), 256, 0, s>>>(*d, sm, sn, sm, 0);
-		}
+	if (tgk_mm_tiled(d)) {
+		launch_mm_tile(s, d, rows);
 		return;
 	}
 	mm_exact_k<<<blocks_for(total), TPB, 0, s>>>(*d, total);

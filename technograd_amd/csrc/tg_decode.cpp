@@ -16,6 +16,7 @@
 #include "tg_kern.h"
 #include "tgm.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -25,6 +26,8 @@
 const tgm_module *tgh_prog_module(const tg_hip_prog *p);
 hipStream_t tgh_prog_stream(const tg_hip_prog *p);
 void tgh_set_error(const char *msg);
+
+constexpr long SC_MAX = 1L << 29; // floats of prompt scores kept for more than one head (2 GiB)
 
 struct tg_hip_dec {
 	const tg_hip_prog *p = nullptr;
@@ -46,6 +49,7 @@ struct tg_hip_dec {
 	long kv_seq = 0;
 	float *ids = nullptr, *h = nullptr, *n = nullptr, *qkv = nullptr, *hq = nullptr, *rt = nullptr;
 	float *qr = nullptr, *att = nullptr, *wout = nullptr, *gu = nullptr, *act = nullptr, *dbuf = nullptr;
+	long sc_floats = 0;  // size of sc, a prompt's scores: all heads' up to SC_MAX, at least one's
 	float *sc = nullptr, *lastn = nullptr, *logits = nullptr;
 	float *am_v = nullptr; // argmax workspace: TGK_AM_PARTS per sequence
 	int *am_i = nullptr;
@@ -234,23 +238,30 @@ bool forward(tg_hip_dec *d, int S, int T0, int p0)
 			a.qr = d->qr, a.K = d->K, a.V = d->Vc, a.att = d->att, a.kv_seq = d->kv_seq, a.kv_layer = kv_layer;
 			a.NQ = d->NQ, a.NKV = d->NKV, a.HD = d->HD, a.P = d->P, a.p = p0, a.scale = d->scale;
 			tgk_dec_attn(st, &a, S);
-		} else { // a prompt from position 0: per head, the graph's products, scale, mask and softmax (causal)
-			for (int hh = 0; hh < d->NQ; hh++) {
-				const int j = hh / GRP;
-				tgk_mm m;
+		} else { // a prompt from position 0: the graph's products, scale, mask and softmax (causal), the heads that
+			// the score buffer holds in one launch (a head alone leaves the chip half empty)
+			const long lines = (long)S * T0;
+			int nh = (int)std::min<long>(d->NQ, d->sc_floats / (lines * T0));
+			if (nh >= GRP) nh -= nh % GRP; // whole KV heads, or heads of one
+			else
+				while (GRP % nh) nh--;
+			for (int h0 = 0, n = 0; h0 < d->NQ; h0 += n) {
+				n = std::min(nh, d->NQ - h0);
+				const long kv = kv_layer + (long)(h0 / GRP) * d->P * d->HD, tt = (long)T0 * T0;
+				tgk_mm m, v;
 				memset(&m, 0, sizeof m);
-				m.g = 1, m.m = T0, m.k = d->HD, m.n = T0, m.causal = 1;
-				m.a = tgk_opd{ d->qr + (long)hh * d->HD, (long)T0 * d->NQ * d->HD }, m.ai = (long)d->NQ * d->HD, m.ap = 1;
-				m.b = tgk_opd{ d->K + kv_layer + (long)j * d->P * d->HD, d->kv_seq }, m.bp = 1, m.bj = d->HD;
-				m.o = d->sc, m.ors = (long)T0 * T0, m.oi = T0, m.oj = 1;
+				m.g = n, m.m = T0, m.k = d->HD, m.n = T0, m.causal = 1, m.gb = std::min(GRP, nh);
+				m.a = tgk_opd{ d->qr + (long)h0 * d->HD, (long)T0 * d->NQ * d->HD }, m.ag = d->HD, m.ai = (long)d->NQ * d->HD, m.ap = 1;
+				m.b = tgk_opd{ d->K + kv, d->kv_seq }, m.bg = (long)d->P * d->HD, m.bp = 1, m.bj = d->HD;
+				m.o = d->sc, m.ors = n * tt, m.og = tt, m.oi = T0, m.oj = 1;
+				memset(&v, 0, sizeof v);
+				v.g = n, v.m = T0, v.k = T0, v.n = d->HD, v.causal = 2, v.gb = m.gb;
+				v.a = tgk_opd{ d->sc, n * tt }, v.ag = tt, v.ai = T0, v.ap = 1;
+				v.b = tgk_opd{ d->Vc + kv, d->kv_seq }, v.bg = m.bg, v.bp = d->HD, v.bj = 1;
+				v.o = d->att + (long)h0 * d->HD, v.ors = (long)T0 * d->NQ * d->HD, v.og = d->HD, v.oi = (long)d->NQ * d->HD, v.oj = 1;
 				tgk_matmul_exact(st, &m, S);
-				tgk_dec_causal_softmax(st, d->sc, T0, (long)S * T0, d->scale);
-				memset(&m, 0, sizeof m);
-				m.g = 1, m.m = T0, m.k = T0, m.n = d->HD, m.causal = 2;
-				m.a = tgk_opd{ d->sc, (long)T0 * T0 }, m.ai = T0, m.ap = 1;
-				m.b = tgk_opd{ d->Vc + kv_layer + (long)j * d->P * d->HD, d->kv_seq }, m.bp = d->HD, m.bj = 1;
-				m.o = d->att + (long)hh * d->HD, m.ors = (long)T0 * d->NQ * d->HD, m.oi = (long)d->NQ * d->HD, m.oj = 1;
-				tgk_matmul_exact(st, &m, S);
+				tgk_dec_causal_softmax(st, d->sc, T0, lines * n, d->scale, tgk_mm_tiled(&v) ? TGK_MM_TILE : 0);
+				tgk_matmul_exact(st, &v, S);
 			}
 		}
 		// a step: all heads in one launch, the same values (heads of at most TGK_REFLOOP_K take the
@@ -355,6 +366,8 @@ bool build(tg_hip_dec *d)
 	if (d->wrot < 0 || d->wlm < 0) return err("decoder: cannot place Rot or the LM head");
 	// cache and buffers
 	const long rows = (long)d->S * d->TP;
+	const long sc1 = (long)d->S * d->TP * d->TP;
+	d->sc_floats = std::max(sc1, std::min(sc1 * d->NQ, SC_MAX));
 	d->kv_seq = (long)d->NKV * d->P * HD; // one sequence's K (or V) of one layer; a layer holds S of them
 	if (!alloc(d, &d->K, (size_t)(d->L * d->S * d->kv_seq)) || !alloc(d, &d->Vc, (size_t)(d->L * d->S * d->kv_seq)) || !alloc(d, &d->ids, (size_t)rows) ||
 	    !alloc(d, &d->h, (size_t)(rows * d->D)) ||
@@ -362,7 +375,7 @@ bool build(tg_hip_dec *d)
 	    !alloc(d, &d->rt, (size_t)(rows * NH * HD)) || !alloc(d, &d->qr, (size_t)(rows * d->NQ * HD)) ||
 	    !alloc(d, &d->att, (size_t)(rows * d->NQ * HD)) || !alloc(d, &d->wout, (size_t)(rows * d->NQ * d->D)) ||
 	    !alloc(d, &d->gu, (size_t)(rows * 2 * d->FF)) || !alloc(d, &d->act, (size_t)(rows * d->FF)) || !alloc(d, &d->dbuf, (size_t)(rows * d->D)) ||
-	    !alloc(d, &d->sc, (size_t)((long)d->S * d->TP * d->TP)) ||
+	    !alloc(d, &d->sc, (size_t)d->sc_floats) ||
 	    !alloc(d, &d->lastn, (size_t)((long)d->S * d->D)) || !alloc(d, &d->logits, (size_t)((long)d->S * d->V)) ||
 	    !alloc(d, &d->am_v, (size_t)d->S * TGK_AM_PARTS) || !alloc(d, &d->am_i, (size_t)d->S * TGK_AM_PARTS))
 		return false;

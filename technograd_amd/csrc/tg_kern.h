@@ -92,7 +92,11 @@ typedef struct {
 	 * i0 .. i0 + TS - 1 sums p = 0 .. i0 + TS - 1 only (the omitted terms add
 	 * +0 to sums that are never -0) */
 	int causal;
+	int gb; /* consecutive groups that share one B (query heads of a KV head); 0 or 1: each has its own */
 } tgk_mm;
+#define TGK_MM_TILE 64
+/* whether an unquantized product runs in 64 x 64 tiles (and takes `causal`) */
+bool tgk_mm_tiled(const tgk_mm *d);
 void tgk_matmul_exact(hipStream_t s, const tgk_mm *d, int rows);
 
 /* softmax (op TGM_SOFTMAX) or rmsnorm over `cols`-long rows, `nrow` of them per batch row */
@@ -218,11 +222,13 @@ void tgk_dec_silu_mul(hipStream_t s, const float *gu, long gus, float *out, int 
  * values equal to the digit + matrix-core path; codes int32 [NQ][HD/4][D],
  * 4 consecutive k's int8 codes per word */
 size_t tgk_dec_wo_lds(int rows, int HD);
-/* one head's causal softmax over a prompt chunk's scores sc [lines][T0]
- * (line L is position L % T0 of its sequence): x = s * scale + 0 and the
- * softmax on u <= t, p = 0 above the diagonal; T0 <= TGK_DEC_PROMPT_MAX */
+/* causal softmax over a prompt chunk's scores sc [lines][T0] (line L is
+ * position L % T0 of its sequence and head): x = s * scale + 0 and the
+ * softmax on u <= t, p = 0 above the diagonal, up to the end of the line's
+ * tile of ztile positions (what a causal tiled product reads; 0: the whole
+ * line); T0 <= TGK_DEC_PROMPT_MAX */
 #define TGK_DEC_PROMPT_MAX 4088 /* 4 lines of T0 + 4 floats in 64 KiB of LDS */
-void tgk_dec_causal_softmax(hipStream_t s, float *sc, int T0, long nlines, float scale);
+void tgk_dec_causal_softmax(hipStream_t s, float *sc, int T0, long nlines, float scale, int ztile);
 void tgk_dec_wo(hipStream_t s, const float *att, const int *codes, const float *scales, float *out, int rows, int NQ, int HD, int D);
 /* pv, pi: TGK_AM_PARTS per row of workspace (each row's parts' best) */
 #define TGK_AM_PARTS 64
