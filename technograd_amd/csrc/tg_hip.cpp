@@ -200,6 +200,12 @@ struct tg_hip_prog {
 	rp_ins *d_rprog = nullptr;
 	long rp_arena = 0;
 	int rp_in_slot = 0, rp_out_ref = 0;
+	// row program run an instruction at a time (run_fixed_steps): per RP_MM its packed weights in d_fxw (-1: two row
+	// values), and the unary instruction after it that its kernel applies
+	bool fx_steps = false;
+	std::vector<long> fx_w;
+	std::vector<char> fx_fused;
+	int *d_fxw = nullptr;
 	// calibration capture (tg_hip_quantize_model): value -> capture index, each capture's axis and per-row sample capacity
 	std::vector<int> cap_of, cap_axis, cap_rows;
 	int cap_both = 0; // a product of two eligible params (both sides would be samples): not captured
@@ -1806,8 +1812,83 @@ void scan_tids(const tgm_block *b, std::vector<std::pair<int, int>> &out)
 	}
 }
 
+tgk_fx fx_opnd(const tg_hip_prog *p, int ref)
+{
+	if (ref >= 0) return tgk_fx{ (const int *)p->d_arena + (long)ref * p->max_rows, p->max_rows, 1 };
+	return tgk_fx{ (const int *)p->d_pool + (-(long)ref - 1), 1, 0 };
+}
+
+// instructions lo .. hi - 1 of a Q16.16 row program over all rows, a launch each; t: the innermost scan's step
+void run_fixed_steps(tg_hip_prog *p, int lo, int hi, int t, int rows, int *d_steps)
+{
+	const hipStream_t st = p->st;
+	const long R = p->max_rows;
+	const int nthink = p->m->nthink ? p->m->nthink : 1;
+	for (int pc = lo; pc < hi; pc++) {
+		const rp_ins &I = p->rprog[(size_t)pc];
+		int *o = (int *)fx_opnd(p, I.out).p;
+		const tgk_fx a = fx_opnd(p, I.a), b = fx_opnd(p, I.b);
+		switch (I.kind) {
+		case RP_BIN:
+			tgk_fx_binary(st, I.op, o, R, a, I.p[0], p->d_imap + I.p[1], b, I.p[2], p->d_imap + I.p[3], I.n, rows);
+			break;
+		case RP_UN:
+			if (!p->fx_fused[(size_t)pc]) tgk_fx_unary(st, I.op, o, R, a, I.n, rows);
+			break;
+		case RP_MM: {
+			const int M = I.p[1], K = I.p[2], N = I.p[3], quant = I.p[4];
+			if (p->fx_w[(size_t)pc] < 0) {
+				tgk_fx_mulrow(st, o, R, a, b, I.p[0], M, K, N, rows);
+				break;
+			}
+			const bool left = quant == 1 || (!quant && I.a < 0); // the weights' side
+			const bool fuse = pc + 1 < (int)p->fx_fused.size() && p->fx_fused[(size_t)pc + 1];
+			tgk_fx_mm d;
+			d.o = fuse ? (int *)fx_opnd(p, p->rprog[(size_t)pc + 1].out).p : o;
+			d.uop = fuse ? p->rprog[(size_t)pc + 1].op : -1;
+			d.R = R;
+			d.w = p->d_fxw + p->fx_w[(size_t)pc];
+			d.qscale = quant ? p->d_qscale + I.p[7] : nullptr;
+			d.x = left ? b : a;
+			d.C = left ? M : N, d.K = K, d.nq = left ? N : M, d.rows = rows;
+			d.xp = left ? N : 1, d.xq = left ? 1 : K;
+			d.oc = left ? N : 1, d.oq = left ? 1 : N;
+			tgk_fx_mul(st, &d);
+			break;
+		}
+		case RP_ROW: tgk_fx_rowop(st, I.op, o, R, a, I.p[0], I.p[1], rows); break;
+		case RP_RED: tgk_fx_reduce(st, I.op, o, a, I.n, rows); break;
+		case RP_TRANS: tgk_fx_transpose(st, o, R, a, I.p[0], I.p[1], I.p[2], rows); break;
+		case RP_OUTER: tgk_fx_outer(st, o, R, a, I.p[0], b, I.p[1], rows); break;
+		case RP_COPY:
+			tgk_fx_copy(st, o, R, I.p[0] + (I.p[3] ? (long)t * I.n : 0), a, I.p[1] + (I.p[2] ? (long)t * I.n : 0), I.n, rows);
+			break;
+		case RP_TAKE: tgk_fx_take(st, o, R, a, b, I.p[0], I.p[1], I.p[2], rows); break;
+		case RP_SCAN: {
+			int end = pc + 1, depth = 1; // its RP_SCAN_END
+			for (;; end++) {
+				if (p->rprog[(size_t)end].kind == RP_SCAN) depth++;
+				if (p->rprog[(size_t)end].kind == RP_SCAN_END && --depth == 0) break;
+			}
+			for (int i = 0; i < I.p[0]; i++) run_fixed_steps(p, pc + 1, end, I.p[1] ? I.p[0] - 1 - i : i, rows, d_steps);
+			if (I.p[2] >= 0 && d_steps) tgk_fx_fill(st, d_steps + I.p[2], nthink, I.p[0], rows);
+			pc = end;
+			break;
+		}
+		default: break;
+		}
+	}
+}
+
 int run_pass(tg_hip_prog *p, const float *d_in, int rows, float *d_out, int *d_steps)
 {
+	if (p->fx_steps) {
+		if (rows <= 0) return 0;
+		tgk_fx_in(p->st, (int *)p->d_arena + (long)p->rp_in_slot * p->max_rows, p->max_rows, (const int *)d_in, (int)p->m->per, rows);
+		run_fixed_steps(p, 0, (int)p->rprog.size(), 0, rows, d_steps);
+		tgk_fx_out(p->st, (int *)d_out, fx_opnd(p, p->rp_out_ref), (int)p->m->nout, rows);
+		return hipok(hipGetLastError(), "fixed program launch") ? 0 : -1;
+	}
 	if (p->executor == 1 && p->rp_fn) {
 		if (rows <= 0) return 0;
 		const void *in = d_in;
@@ -2237,6 +2318,74 @@ bool compile_rowprog(tg_hip_prog *p, const RB &B, bool &fatal)
 	return true;
 }
 
+// A Q16.16 program that the compiler refuses and that has no think loop runs
+// an instruction at a time over all rows (kern_fixed.hip), unless the
+// interpreter or the one-lane-per-row form was asked for, or its scans run
+// bodies of a few values. Products with a
+// quantized or f32 param keep its weights as one int32 word each, 16
+// channels side by side.
+bool plan_fixed_steps(tg_hip_prog *p, const RB &B)
+{
+	if (!p->fixed || (p->flags & (TG_HIP_INTERP | TG_HIP_ROWPROG))) return true;
+	const auto &Pr = p->rprog;
+	double terms = 0, launches = 0, mult = 1; // of one row, of a pass (scan bodies as often as they run)
+	std::vector<double> outer;
+	for (const rp_ins &I : Pr) {
+		if (I.kind == RP_THINK) return true;
+		if (I.kind == RP_SCAN) outer.push_back(mult), mult *= I.p[0];
+		else if (I.kind == RP_SCAN_END) mult = outer.back(), outer.pop_back();
+		else launches += mult;
+		if (I.kind == RP_MM) terms += mult * I.p[0] * I.p[1] * I.p[2] * I.p[3];
+		else if (I.kind == RP_ROW || I.kind == RP_OUTER) terms += mult * I.p[0] * I.p[1];
+		else if (I.kind == RP_TRANS || I.kind == RP_TAKE) terms += mult * I.p[0] * (I.kind == RP_TRANS ? I.p[1] : 1) * I.p[2];
+		else terms += mult * I.n;
+	}
+	// The interpreter takes 0.15-0.3 us a term (one lane's chain of loads), a launch about 2.5 us: 41 terms a launch
+	// (a small scan, 32 steps) 5.2 ms against 1.15, so it keeps what does fewer than 16.
+	if (terms < 16 * launches) return true;
+	p->fx_w.assign(Pr.size(), -1);
+	p->fx_fused.assign(Pr.size(), 0);
+	std::vector<int> w;
+	std::map<std::vector<int>, long> have; // a param's packing, shared by the products that read it
+	for (size_t i = 0; i < Pr.size(); i++) {
+		const rp_ins &I = Pr[i];
+		if (I.kind != RP_MM || I.p[0] != 1) continue;
+		const int M = I.p[1], K = I.p[2], N = I.p[3], quant = I.p[4];
+		if (!quant && (I.a < 0) == (I.b < 0)) continue; // two row values (or two params: the row form reads both)
+		const bool left = quant == 1 || (!quant && I.a < 0);
+		const int C = left ? M : N;
+		const std::vector<int> key{ left, quant, quant ? I.p[6] : left ? I.a : I.b, M, K, N };
+		auto it = have.find(key);
+		if (it == have.end()) {
+			it = have.emplace(key, (long)w.size()).first;
+			w.resize(w.size() + (size_t)((C + 15) / 16) * K * 16, 0);
+			int *dst = w.data() + it->second;
+			for (int c = 0; c < C; c++)
+				for (int k = 0; k < K; k++) {
+					const long e = left ? (long)c * K + k : (long)k * N + c;
+					int v;
+					if (quant) {
+						const uint8_t *q = B.P.codes.data() + I.p[6];
+						v = I.p[5] == 8 ? (int)(int8_t)q[e] : (int)(int8_t)(uint8_t)(q[e >> 1] << (e & 1 ? 0 : 4)) >> 4;
+					} else {
+						memcpy(&v, &B.P.f[(size_t)(-(long)(left ? I.a : I.b) - 1 + e)], 4);
+					}
+					dst[((size_t)(c / 16) * K + k) * 16 + c % 16] = v;
+				}
+		}
+		p->fx_w[i] = it->second;
+		// a unary instruction right after it that alone reads the product, elementwise
+		if (i + 1 < Pr.size() && Pr[i + 1].kind == RP_UN && Pr[i + 1].a == I.out && Pr[i + 1].n == M * N && p->rp_out_ref != I.out) {
+			bool alone = true;
+			for (size_t j = 0; j < Pr.size(); j++)
+				if (j != i + 1 && (Pr[j].a == I.out || Pr[j].b == I.out) && Pr[j].kind != RP_SCAN && Pr[j].kind != RP_SCAN_END) alone = false;
+			p->fx_fused[i + 1] = alone;
+		}
+	}
+	p->fx_steps = true;
+	return upload(&p->d_fxw, w, p->st) && hipok(hipStreamSynchronize(p->st), "upload");
+}
+
 bool build_rowprog(tg_hip_prog *p)
 {
 	RB B;
@@ -2249,6 +2398,7 @@ bool build_rowprog(tg_hip_prog *p)
 		p->rp_why = "the interpreter was requested (TG_HIP_INTERP)";
 	}
 	if (!upload_pools(p, B.P) || !upload(&p->d_rprog, p->rprog, p->st)) return false;
+	if (!plan_fixed_steps(p, B)) return false;
 	size_t ab = (size_t)p->rp_arena * p->max_rows * sizeof(float);
 	p->stats.arena_bytes = (long)ab;
 	return hipok(hipMalloc(&p->d_arena, ab), "arena") && hipok(hipStreamSynchronize(p->st), "upload");
@@ -2258,7 +2408,7 @@ void destroy(tg_hip_prog *p)
 {
 	if (!p) return;
 	for (auto &q : p->qws) tgk_qweight_free(&q);
-	void *bufs[] = { p->d_pool, p->d_imap, p->d_codes, p->d_fscale, p->d_qscale, p->d_arena, p->d_scratch, p->d_rprog, p->d_steps,
+	void *bufs[] = { p->d_pool, p->d_imap, p->d_codes, p->d_fscale, p->d_qscale, p->d_arena, p->d_scratch, p->d_rprog, p->d_steps, p->d_fxw,
 		         p->d_cap, p->d_cap_base, p->d_cap_k, p->d_cap_rows, p->d_cap_count };
 	for (void *b : bufs)
 		if (b) (void)hipFree(b);

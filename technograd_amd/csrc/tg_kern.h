@@ -367,6 +367,43 @@ typedef struct {
 } rp_args;
 
 void tgk_rowprog(hipStream_t s, const rp_args *a);
+
+/* ---- Q16.16 row programs an instruction at a time (kern_fixed.hip) ---- */
+
+/* a row program's operand: element i of row r at p[i st + r ls] (arena values
+ * st = R, ls = 1; pool values st = 1, ls = 0); outputs are arena values, R apart */
+typedef struct {
+	const int *p;
+	long st, ls;
+} tgk_fx;
+/* o element c oc + q oq = uop(finish(sum_p w[c][p] x element p xp + q xq)) for
+ * C channels and nq inner positions; w packed [ceil(C/16)][K][16] int32 (zeros
+ * past C), finish the Q7.24 scale qscale[c], or the Q16 rounding when NULL;
+ * uop a unary TGM_ op, or -1 */
+typedef struct {
+	int *o;
+	long R, oc, oq;
+	const int *w;
+	const int *qscale;
+	tgk_fx x;
+	long xp, xq;
+	int C, K, nq, rows, uop;
+} tgk_fx_mm;
+void tgk_fx_mul(hipStream_t s, const tgk_fx_mm *d);
+void tgk_fx_mulrow(hipStream_t s, int *o, long R, tgk_fx a, tgk_fx b, int G, int M, int K, int N, int rows);
+void tgk_fx_binary(hipStream_t s, int op, int *o, long R, tgk_fx a, int am, const int *amap, tgk_fx b, int bm, const int *bmap, int n, int rows);
+void tgk_fx_unary(hipStream_t s, int op, int *o, long R, tgk_fx a, int n, int rows);
+void tgk_fx_rowop(hipStream_t s, int op, int *o, long R, tgk_fx a, int nrow, int cols, int rows);
+void tgk_fx_reduce(hipStream_t s, int op, int *o, tgk_fx a, int n, int rows);
+void tgk_fx_transpose(hipStream_t s, int *o, long R, tgk_fx a, int g, int r, int c, int rows);
+void tgk_fx_outer(hipStream_t s, int *o, long R, tgk_fx a, int m, tgk_fx b, int n, int rows);
+void tgk_fx_copy(hipStream_t s, int *o, long R, long ooff, tgk_fx a, long aoff, int n, int rows);
+void tgk_fx_take(hipStream_t s, int *o, long R, tgk_fx w, tgk_fx idx, int cnt, int d, int h, int rows);
+void tgk_fx_fill(hipStream_t s, int *o, int stride, int v, int rows);
+/* [rows][n] <-> arena values */
+void tgk_fx_in(hipStream_t s, int *o, long R, const int *in, int n, int rows);
+void tgk_fx_out(hipStream_t s, int *out, tgk_fx a, int n, int rows);
+
 /* H[r][c] = sum over the rows in order, then each row's samples in order, of
  * x_r x_c in f64 (the order of the reference's hook): capture c of a pass */
 void tgk_hessian(hipStream_t s, const float *cap, const int *count, long row_cap, int K, int rows, double *H);
