@@ -193,199 +193,6 @@ __global__ __launch_bounds__(ATT_TPB) void dec_attn_k(tgk_dec_attn_args a, int c
 	}
 }
 
-// The per-head output projections of a decode step, all heads in one launch:
-// out[g][t][c] = x_{t,g} @ W_g[:, c] for query head g, token t, x_{t,g} the
-// head's attention output [HD]. Each value is the one the digit kernel and
-// the matrix-core GEMM produce for that row: the row's exponent E from its
-// max |x| (bumped when the top digit would overflow), q_k = rint(x_k 2^(23-E))
-// exactly, split into the same three balanced int8 digits, the exact integer
-// sum_k code_k q_k = s0 + 256 s1 + 65536 s2 (s_i = sum_k code_k digit_i,k by
-// 4-way int8 dot products), scaled by 2^(E-23) in f64, rounded once to f32
-// and multiplied by the channel scale; rows with inf, nan or an entry above
-// 2^100 take the reference's sequential f32 loop, and candidate rows
-// (tg_qdigits.h) are resolved here as the GEMM path resolves them: a wave
-// per row, the same decision; a split row's rest gets digits of its own
-// grid and its outliers' terms (f64, increasing k) are added to its grid
-// sum before the one rounding. One block per (head, 64 columns): the rows'
-// digits and the head's code tile sit in LDS; a wave handles 4 rows at a
-// time, a lane one column.
-// codes: int32 [NQ][HD/4][D], 4 consecutive k's int8 codes per word (k = 4
-// k4 + i in byte i); scales [NQ][D]; HD a multiple of 4, att 16-byte aligned.
-constexpr int WO_TPB = 512, WO_NW = WO_TPB / 64;
-constexpr int wo_nout(int HD) { return HD / 16 < 1 ? 1 : HD / 16 > TGQ_MAX_OUT ? TGQ_MAX_OUT : HD / 16; } // >= J(n), n <= HD
-__global__ __launch_bounds__(WO_TPB) void dec_wo_k(const float *att, const int *codes, const float *scales, float *out, int rows, int NQ,
-						   int HD, int D)
-{
-	extern __shared__ int4 dg[]; // [rows][HD/4] digit words {d0, d1, d2, 0} of 4 k's
-	const int H4 = HD / 4, n = rows * H4, NO = wo_nout(HD);
-	TgqHist *hist = (TgqHist *)(dg + (long)rows * H4); // one per wave
-	long long *tq = (long long *)(hist + WO_NW);      // per row: the candidate tally
-	float *ox = (float *)(tq + rows);                 // per row: a split row's outliers [NO], values
-	int *ok = (int *)(ox + (long)rows * NO);          // and inputs, -1 past the last
-	int *Es = ok + (long)rows * NO, *sp = Es + rows, *ct = sp + rows; // ct: [HD/4][64] code words
-	const int ctiles = (D + 63) / 64, g = blockIdx.x / ctiles, c0 = (blockIdx.x - g * ctiles) * 64;
-	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-	constexpr int U = 4;
-	auto xat = [&](int e) { // the 4 inputs of item e = (row t, k4)
-		const int t = e / H4;
-		return *(const float4 *)(att + ((long)t * NQ + g) * HD + 4 * (e - t * H4));
-	};
-	// rows' max |x| (as bits: non-negative floats order as their bits) and flags
-	unsigned *mxb = (unsigned *)Es;
-	for (int t = tid; t < rows; t += WO_TPB) mxb[t] = 0, sp[t] = 0, tq[t] = 0;
-	for (int e = tid; e < H4 * 64; e += WO_TPB) {
-		const int k4 = e >> 6, c = e & 63;
-		ct[e] = c0 + c < D ? codes[((long)g * H4 + k4) * D + c0 + c] : 0;
-	}
-	__syncthreads();
-	for (int b = tid; b < n; b += U * WO_TPB) {
-		float4 u[U];
-		for (int j = 0; j < U; j++) u[j] = xat(min(b + j * WO_TPB, n - 1));
-		for (int j = 0; j < U; j++) {
-			const int e = b + j * WO_TPB;
-			if (e >= n) continue;
-			const float4 v = u[j];
-			const int bad = !isfinite(v.x) || !isfinite(v.y) || !isfinite(v.z) || !isfinite(v.w);
-			const float m = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))); // a nan never wins fmaxf
-			atomicMax(&mxb[e / H4], __float_as_uint(m));
-			if (bad) atomicOr(&sp[e / H4], 1);
-		}
-	}
-	__syncthreads();
-	for (int t = tid; t < rows; t += WO_TPB) {
-		const float mx = __uint_as_float(mxb[t]);
-		const int special = tgq_special(sp[t], mx);
-		Es[t] = tgq_exponent(mx, special), sp[t] = special;
-	}
-	__syncthreads();
-	// the four inputs' digit words on the grid of E; their tally into *tl
-	auto digit_words = [&](const float (&xv)[4], int E, long long *tl) {
-		unsigned w0 = 0, w1 = 0, w2 = 0;
-		int aq = 0, nx = 0;
-		for (int i = 0; i < 4; i++) {
-			const float sv = ldexpf(xv[i], 23 - E), rq = rintf(sv);
-			const int q = (int)rq; // exact: |q| < 2^23
-			aq += abs(q);
-			nx += rq != sv;
-			int d0, d1, d2;
-			tgq_split3(q, d0, d1, d2);
-			w0 |= (unsigned)(d0 & 255) << (8 * i);
-			w1 |= (unsigned)(d1 & 255) << (8 * i);
-			w2 |= (unsigned)(d2 & 255) << (8 * i);
-		}
-		if (tl && (aq || nx)) atomicAdd((unsigned long long *)tl, (unsigned long long)aq + ((unsigned long long)nx << TGQ_TALLY_SHIFT));
-		return make_int4((int)w0, (int)w1, (int)w2, 0);
-	};
-	for (int b = tid; b < n; b += U * WO_TPB) {
-		float4 u[U];
-		for (int j = 0; j < U; j++) u[j] = xat(min(b + j * WO_TPB, n - 1));
-		for (int j = 0; j < U; j++) {
-			const int e = b + j * WO_TPB;
-			if (e >= n) continue;
-			const int t = e / H4;
-			const float xv[4] = { u[j].x, u[j].y, u[j].z, u[j].w };
-			dg[e] = sp[t] ? make_int4(0, 0, 0, 0) : digit_words(xv, Es[t], &tq[t]);
-		}
-	}
-	__syncthreads();
-	for (int t = tid; t < rows; t += WO_TPB)
-		if (!sp[t] && tgq_candidate(tq[t])) sp[t] = 3; // a candidate, resolved below
-	__syncthreads();
-	// candidates: a wave per row, the GEMM path's resolve (kern_qgemm.hip: resolve_k)
-	for (int t = wave; t < rows; t += WO_NW) {
-		if (sp[t] != 3) continue; // the same word for the whole wave
-		const float *x = att + ((long)t * NQ + g) * HD;
-		const int E0 = Es[t];
-		auto ld = [&](int gi, float *v) {
-			for (int i = 0; i < 16; i++) v[i] = 16 * gi + i < HD ? x[16 * gi + i] : 0.0f;
-		};
-		TgqCoarse co{}; // the coarse test first (tg_qdigits.h)
-		for (int gi = lane; gi < (HD + 15) / 16; gi += 64) {
-			float v[16];
-			ld(gi, v);
-			tgq_coarse16(co, v, E0);
-		}
-		if (tgq_coarse_grid(tgq_coarse_wave_sum(co), tq[t])) {
-			if (lane == 0) sp[t] = 0;
-			continue;
-		}
-		const int L = tgq_resolve(&hist[wave], ld, (HD + 15) / 16, E0, lane);
-		if (L <= 0) {
-			if (lane == 0) sp[t] = L < 0 ? 1 : 0;
-			continue;
-		}
-		float rm = 0.0f;
-		for (int k = lane; k < HD; k += 64)
-			if (!tgq_outlier(x[k], E0, L)) rm = fmaxf(rm, fabsf(x[k]));
-		for (int o = 32; o > 0; o >>= 1) rm = fmaxf(rm, __shfl_xor(rm, o));
-		const int Er = tgq_exponent(rm, 0);
-		int nin = 0;
-		for (int k40 = 0; k40 < H4; k40 += 64) { // the rest's digits, the outliers in input order
-			const int k4 = k40 + lane;
-			float xv[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
-			unsigned om = 0;
-			if (k4 < H4)
-				for (int i = 0; i < 4; i++) {
-					const float xi = x[4 * k4 + i];
-					if (tgq_outlier(xi, E0, L)) om |= 1u << i;
-					else xv[i] = xi;
-				}
-			if (k4 < H4) dg[(long)t * H4 + k4] = digit_words(xv, Er, nullptr);
-			const int cnt = __popc(om);
-			int inc = cnt;
-			for (int d = 1; d < 64; d <<= 1) {
-				const int y = __shfl_up(inc, d);
-				if (lane >= d) inc += y;
-			}
-			int at = nin + inc - cnt;
-			for (int i = 0; i < 4; i++)
-				if ((om >> i) & 1) {
-					if (at < NO) ok[(long)t * NO + at] = 4 * k4 + i, ox[(long)t * NO + at] = x[4 * k4 + i];
-					at++;
-				}
-			nin += __shfl(inc, 63);
-		}
-		for (int j = nin + lane; j < NO; j += 64) ok[(long)t * NO + j] = -1;
-		if (lane == 0) Es[t] = Er, sp[t] = 2;
-	}
-	__syncthreads();
-	const int c = lane;
-	if (c0 + c >= D) return;
-	const float sc = scales[(long)g * D + c0 + c];
-	for (int t0 = 4 * wave; t0 < rows; t0 += 4 * WO_NW) {
-		int s[4][3] = {};
-		int tr[4];
-		for (int r = 0; r < 4; r++) tr[r] = min(t0 + r, rows - 1); // rows past the end repeat the last (not stored)
-		for (int k4 = 0; k4 < H4; k4++) {
-			const int w = ct[k4 * 64 + c];
-			for (int r = 0; r < 4; r++) {
-				const int4 d = dg[(long)tr[r] * H4 + k4];
-				s[r][0] = __builtin_amdgcn_sdot4(w, d.x, s[r][0], false);
-				s[r][1] = __builtin_amdgcn_sdot4(w, d.y, s[r][1], false);
-				s[r][2] = __builtin_amdgcn_sdot4(w, d.z, s[r][2], false);
-			}
-		}
-		for (int r = 0; r < 4 && t0 + r < rows; r++) {
-			const int t = t0 + r;
-			auto code = [&](int k) { return (float)(int8_t)(ct[(k >> 2) * 64 + c] >> (8 * (k & 3))); };
-			float v;
-			if (sp[t] == 1) { // the reference's loop (runtime/tg_rt.h:143-151)
-				const float *x = att + ((long)t * NQ + g) * HD;
-				float acc = 0.0f;
-				for (int k = 0; k < HD; k++) acc += code(k) * x[k];
-				v = acc;
-			} else { // every term and partial sum an integer below 2^48: exact in f64
-				const double tot = (double)s[r][0] + (double)s[r][1] * 256.0 + (double)s[r][2] * 65536.0;
-				double o = 0.0; // a split row's outlier terms, in input order
-				if (sp[t] == 2)
-					for (int j = 0; j < NO && ok[(long)t * NO + j] >= 0; j++) o += (double)code(ok[(long)t * NO + j]) * (double)ox[(long)t * NO + j];
-				v = (float)(ldexp(tot, Es[t] - 23) + o);
-			}
-			out[((long)g * rows + t) * D + c0 + c] = sc * v;
-		}
-	}
-}
-
 // Block-wide reductions (blockDim a multiple of 64, at most 1024); red is
 // LDS scratch of 16 entries. Every thread gets the result.
 __device__ inline float blk_max(float v, float *red)
@@ -1027,16 +834,6 @@ void tgk_dec_causal_softmax(hipStream_t s, float *sc, int T0, long nlines, float
 	const size_t lds = (size_t)lpb * stride * 4 + lpb * 4;
 	if (T0 % 4 == 0 && ((size_t)sc & 15) == 0) causal_softmax_k<4><<<grid, 256, lds, s>>>(sc, T0, nlines, scale, ztile ? ztile : T0, lpb, stride);
 	else causal_softmax_k<1><<<grid, 256, lds, s>>>(sc, T0, nlines, scale, ztile ? ztile : T0, lpb, stride);
-}
-
-size_t tgk_dec_wo_lds(int rows, int HD)
-{
-	return (size_t)rows * HD * 4 + WO_NW * sizeof(TgqHist) + (size_t)rows * (8 + 8 * wo_nout(HD) + 8) + (size_t)HD * 64;
-}
-
-void tgk_dec_wo(hipStream_t s, const float *att, const int *codes, const float *scales, float *out, int rows, int NQ, int HD, int D)
-{
-	if (rows > 0) dec_wo_k<<<(unsigned)(NQ * ((D + 63) / 64)), WO_TPB, tgk_dec_wo_lds(rows, HD), s>>>(att, codes, scales, out, rows, NQ, HD, D);
 }
 
 void tgk_dec_argmax(hipStream_t s, const float *x, long xrs, int V, int rows, float *idf, int *idi, long idi_stride, float *pv, int *pi)

@@ -40,9 +40,7 @@ struct tg_hip_dec {
 	// params
 	const float *E = nullptr, *lnf = nullptr, *cosT = nullptr, *sinT = nullptr;
 	std::vector<const float *> ln1, ln2, qkg;
-	std::vector<int> wqkv, wgu, wd, wo; // indices into ws (wo: L x NQ)
-	std::vector<const int *> wo_codes;  // per layer: all heads' output projections for a step, int32 [NQ][HD/4][D]
-	std::vector<const float *> wo_scales; // per layer: [NQ][D]
+	std::vector<int> wqkv, wgu, wd, wo; // indices into ws (wo: one per layer when heads_fused, else L x NQ)
 	int wrot = -1, wlm = -1;
 	// cache and work buffers
 	float *K = nullptr, *Vc = nullptr;
@@ -108,29 +106,24 @@ bool upload(tg_hip_dec *d, const float **dst, const float *src, size_t n)
 	return hip_ok(hipMemcpyAsync(q, src, n * sizeof(float), hipMemcpyHostToDevice, d->st), "decoder upload");
 }
 
-// one layer's per-head output projections W_h [HD][D] (axis-1 scales) as
-// the step kernel's code words: int32 [NQ][HD/4][D], codes of k = 4 k4 .. 4 k4
-// + 3 in bytes 0 .. 3 of word (h, k4, c); scales [NQ][D]
-bool pack_heads(tg_hip_dec *d, const tgm_module *m, const std::vector<int> &vs, const int **codes, const float **scales)
+// one layer's per-head output projections W_h [HD][D] as tgk_heads' weight:
+// int8 codes, head h's channels from h Dp on
+int pack_heads(tg_hip_dec *d, const tgm_module *m, const std::vector<int> &vs)
 {
-	const int HD = d->HD, D = d->D, NQ = (int)vs.size();
-	std::vector<int> w((size_t)NQ * (HD / 4) * D, 0);
-	std::vector<float> sc((size_t)NQ * D);
+	const int HD = d->HD, D = d->D, NQ = (int)vs.size(), Dp = (D + 255) / 256 * 256;
+	std::vector<int8_t> codes((size_t)NQ * Dp * HD, 0);
+	std::vector<float> sc((size_t)NQ * Dp, 0.0f);
 	for (int h = 0; h < NQ; h++) {
 		const tgm_value &x = m->val[vs[(size_t)h]];
-		if (x.sh.rank != 2 || x.sh.dim[0] != HD || x.sh.dim[1] != D || !x.qbits || x.qaxis != 1) return false;
-		for (int k = 0; k < HD; k++)
-			for (int c = 0; c < D; c++) {
-				const unsigned b = (unsigned)(tgm_code(&x, (long)k * D + c) & 255);
-				w[((size_t)h * (HD / 4) + k / 4) * D + c] |= (int)(b << (8 * (k % 4)));
-			}
-		memcpy(&sc[(size_t)h * D], x.qs, (size_t)D * sizeof(float));
+		if (x.sh.rank != 2 || x.sh.dim[0] != HD || x.sh.dim[1] != D || !x.qbits || x.qaxis != 1) return -1;
+		for (int c = 0; c < D; c++)
+			for (int k = 0; k < HD; k++) codes[((size_t)h * Dp + c) * HD + k] = (int8_t)tgm_code(&x, (long)k * D + c);
+		memcpy(&sc[(size_t)h * Dp], x.qs, (size_t)D * sizeof(float));
 	}
-	int *q;
-	if (!alloc(d, &q, w.size()) || !hip_ok(hipMemcpyAsync(q, w.data(), w.size() * sizeof(int), hipMemcpyHostToDevice, d->st), "decoder upload"))
-		return false;
-	*codes = q;
-	return upload(d, scales, sc.data(), sc.size());
+	tgk_qweight w;
+	if (tgk_qweight_pack_i8(&w, codes.data(), sc.data(), 8, NQ * Dp, HD, d->st)) return -1;
+	d->ws.push_back(w);
+	return (int)d->ws.size() - 1;
 }
 
 // pack params (each [K][C_i], quantized on axis 1, x @ W) concatenated along C
@@ -194,6 +187,9 @@ bool gemm_pre(tg_hip_dec *d, int wi, const float *x, long xr, int ni, long xj, i
 	tgk_qgemm_mfma(d->st, &a, d->scratch);
 	return true;
 }
+
+// whether all heads' output projections run as one product (tgk_heads)
+bool heads_fused(const tg_hip_dec *d) { return d->HD > TGK_REFLOOP_K && d->HD <= TGK_HEADS_MAX && d->NQ <= 64; }
 
 // the graph's rmsnorm-then-gain of token rows, fused with the update of h
 // before it (mode 1: h += add; mode 2: h += the heads' output projections in
@@ -264,16 +260,21 @@ bool forward(tg_hip_dec *d, int S, int T0, int p0)
 				tgk_matmul_exact(st, &v, S);
 			}
 		}
-		// a step: all heads in one launch, the same values (heads of at most TGK_REFLOOP_K take the
-		// reference's loop, as every short product does: the per-head products below)
-		if (T0 == 1 && d->HD > TGK_REFLOOP_K && tgk_dec_wo_lds(rows, d->HD) <= 65536)
-			tgk_dec_wo(st, d->att, d->wo_codes[(size_t)l], d->wo_scales[(size_t)l], d->wout, rows, d->NQ, d->HD, d->D);
-		else
+		// h + the heads' output projections (in head order), rmsnorm * ln2, gate and up projections. Heads of at most
+		// TGK_REFLOOP_K take the reference's loop, as every short product does: a product per head, summed by the norm
+		if (heads_fused(d)) {
+			tgk_heads_args ha;
+			ha.x = d->att, ha.xrow = (long)d->NQ * d->HD, ha.xhead = d->HD, ha.rows = rows, ha.rp = (rows + 31) / 32 * 32;
+			ha.nh = d->NQ, ha.HD = d->HD, ha.D = d->D, ha.Dp = (d->D + 255) / 256 * 256;
+			ha.w = &d->ws[(size_t)d->wo[(size_t)l]], ha.o = d->dbuf, ha.orow = D;
+			tgk_heads(st, &ha, d->scratch);
+			res = norm(d, 1, d->h, D, rows, d->dbuf, D, d->ln2[(size_t)l], d->n, d->wgu[(size_t)l]);
+		} else {
 			for (int hh = 0; hh < d->NQ; hh++)
 				gemm(d, d->wo[(size_t)l * d->NQ + hh], d->att + (long)hh * d->HD, (long)d->NQ * d->HD, 1, 0, rows,
 				     d->wout + (long)hh * rows * D, D, 0);
-		// h + the heads' output projections (in head order), rmsnorm * ln2, gate and up projections
-		res = norm(d, 2, d->h, D, rows, nullptr, 0, d->ln2[(size_t)l], d->n, d->wgu[(size_t)l]);
+			res = norm(d, 2, d->h, D, rows, nullptr, 0, d->ln2[(size_t)l], d->n, d->wgu[(size_t)l]);
+		}
 		gemm_pre(d, d->wgu[(size_t)l], d->n, D, 1, 0, rows, d->gu, 2L * d->FF, 0, res);
 		if (rows >= TGK_DEC_SILU_FUSED_MAX) { // a prompt's many rows: act = silu(g) * u streamed, the down projection's own digits
 			tgk_dec_silu_mul(st, d->gu, 2L * d->FF, d->act, d->FF, rows);
@@ -352,14 +353,14 @@ bool build(tg_hip_dec *d)
 		std::vector<int> wo;
 		for (int h = 0; h < d->NQ; h++) {
 			const int v = find(m, nm("Wo_%d_%d", l, h));
-			const int i = v < 0 ? -1 : pack_concat(d, m, { v });
-			if (i < 0) return err("decoder: cannot place layer %s%ld's output projections", "", l);
-			d->wo.push_back(i), wo.push_back(v);
+			if (v < 0) return err("decoder: cannot place layer %s%ld's output projections", "", l);
+			wo.push_back(v);
 		}
-		const int *woc = nullptr;
-		const float *wos = nullptr;
-		if (!pack_heads(d, m, wo, &woc, &wos)) return err("decoder: cannot place layer %s%ld's output projections", "", l);
-		d->wo_codes.push_back(woc), d->wo_scales.push_back(wos);
+		for (int h = 0; h < (heads_fused(d) ? 1 : d->NQ); h++) {
+			const int i = heads_fused(d) ? pack_heads(d, m, wo) : pack_concat(d, m, { wo[(size_t)h] });
+			if (i < 0) return err("decoder: cannot place layer %s%ld's output projections", "", l);
+			d->wo.push_back(i);
+		}
 	}
 	d->wrot = pack_concat(d, m, { vRot });
 	d->wlm = pack_concat(d, m, { vLM });
@@ -373,7 +374,8 @@ bool build(tg_hip_dec *d)
 	    !alloc(d, &d->h, (size_t)(rows * d->D)) ||
 	    !alloc(d, &d->n, (size_t)(rows * d->D)) || !alloc(d, &d->qkv, (size_t)(rows * ctot)) || !alloc(d, &d->hq, (size_t)(rows * NH * HD)) ||
 	    !alloc(d, &d->rt, (size_t)(rows * NH * HD)) || !alloc(d, &d->qr, (size_t)(rows * d->NQ * HD)) ||
-	    !alloc(d, &d->att, (size_t)(rows * d->NQ * HD)) || !alloc(d, &d->wout, (size_t)(rows * d->NQ * d->D)) ||
+	    !alloc(d, &d->att, (size_t)((rows + 31) / 32 * 32 * d->NQ * HD)) ||
+	    !alloc(d, &d->wout, heads_fused(d) ? 0 : (size_t)(rows * d->NQ * d->D)) ||
 	    !alloc(d, &d->gu, (size_t)(rows * 2 * d->FF)) || !alloc(d, &d->act, (size_t)(rows * d->FF)) || !alloc(d, &d->dbuf, (size_t)(rows * d->D)) ||
 	    !alloc(d, &d->sc, (size_t)d->sc_floats) ||
 	    !alloc(d, &d->lastn, (size_t)((long)d->S * d->D)) || !alloc(d, &d->logits, (size_t)((long)d->S * d->V)) ||
@@ -381,8 +383,10 @@ bool build(tg_hip_dec *d)
 		return false;
 	size_t sb = 0;
 	auto need = [&](long M, int wi) { sb = std::max(sb, tgk_qgemm_scratch((int)M, d->ws[(size_t)wi].Kp)); };
-	need(rows, d->wqkv[0]), need(rows * NH, d->wrot), need(rows, d->wo[0]), need(rows, d->wgu[0]), need(rows, d->wd[0]), need(d->S, d->wlm);
+	const long rp = (rows + 31) / 32 * 32; // (tgk_heads reads whole blocks of 32 rows)
+	need(rows, d->wqkv[0]), need(rows * NH, d->wrot), need(heads_fused(d) ? rp * d->NQ : rows, d->wo[0]), need(rows, d->wgu[0]), need(rows, d->wd[0]), need(d->S, d->wlm);
 	d->scratch_bytes = sb;
+	if (!hip_ok(hipMemsetAsync(d->att, 0, (size_t)(rp * d->NQ * HD) * sizeof(float), d->st), "decoder memory")) return false; // (its padding rows are read)
 	return hip_ok(hipMalloc(&d->scratch, sb), "decoder scratch") && hip_ok(hipStreamSynchronize(d->st), "decoder upload");
 }
 

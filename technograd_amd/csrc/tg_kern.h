@@ -218,10 +218,23 @@ bool tgk_dec_silu(hipStream_t s, const tgk_dec_silu_args *a);
  * GEMM after it makes the digits with its own many-row digit kernel */
 void tgk_dec_silu_mul(hipStream_t s, const float *gu, long gus, float *out, int FF, int rows);
 #define TGK_DEC_SILU_FUSED_MAX 512 /* rows below which tgk_dec_silu's one block per row makes the digits */
-/* per-head output projections of `rows` token rows, all heads in one launch,
- * values equal to the digit + matrix-core path; codes int32 [NQ][HD/4][D],
- * 4 consecutive k's int8 codes per word */
-size_t tgk_dec_wo_lds(int rows, int HD);
+/* All heads' output projections of `rows` token rows, the heads added in
+ * order (kern_heads.hip): o[row][c] = ((o_0 + o_1) + ...), o_h the quantized
+ * product of x[row][h] (at row xrow + h xhead, HD values) with head h's
+ * weights. w: int8 codes (whatever the model's width), channel h Dp + c for
+ * (head h, channel c), Dp = D padded to 256 with zero codes. rp: the rows
+ * padded to 32; the x of padding rows is read and dropped. scratch:
+ * tgk_qgemm_scratch(nh rp, w->Kp) bytes. TGK_REFLOOP_K < HD <= TGK_HEADS_MAX, nh <= 64. */
+#define TGK_HEADS_MAX 256
+typedef struct {
+	const float *x;
+	long xrow, xhead;
+	int rows, rp, nh, HD, D, Dp;
+	const tgk_qweight *w;
+	float *o;
+	long orow;
+} tgk_heads_args;
+void tgk_heads(hipStream_t s, const tgk_heads_args *a, void *scratch);
 /* causal softmax over a prompt chunk's scores sc [lines][T0] (line L is
  * position L % T0 of its sequence and head): x = s * scale + 0 and the
  * softmax on u <= t, p = 0 above the diagonal, up to the end of the line's
@@ -229,7 +242,6 @@ size_t tgk_dec_wo_lds(int rows, int HD);
  * line); T0 <= TGK_DEC_PROMPT_MAX */
 #define TGK_DEC_PROMPT_MAX 4088 /* 4 lines of T0 + 4 floats in 64 KiB of LDS */
 void tgk_dec_causal_softmax(hipStream_t s, float *sc, int T0, long nlines, float scale, int ztile);
-void tgk_dec_wo(hipStream_t s, const float *att, const int *codes, const float *scales, float *out, int rows, int NQ, int HD, int D);
 /* pv, pi: TGK_AM_PARTS per row of workspace (each row's parts' best) */
 #define TGK_AM_PARTS 64
 void tgk_dec_argmax(hipStream_t s, const float *x, long xrs, int V, int rows, float *idf, int *idi, long idi_stride, float *pv, int *pi);
