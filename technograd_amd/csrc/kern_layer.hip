@@ -295,8 +295,8 @@ __global__ void rowop_k(int op, float *o, long ors, tgk_opd a, int nrow, int col
 }
 
 // The same per-line results with the lines staged through LDS: a block takes
-// lpb consecutive lines of one batch row (lpb divides nrow), which are
-// contiguous in memory, so loads and stores are coalesced. Only the sums
+// up to lpb consecutive lines of one batch row (its last block what is left),
+// which are contiguous in memory, so loads and stores are coalesced. Only the sums
 // keep one thread per line, walking its line in the reference's order; the
 // max, the exponentials, the division and the rmsnorm scaling are
 // elementwise or order-free and use every thread. LDS lines are `stride`
@@ -319,8 +319,8 @@ __global__ __launch_bounds__(256) void rowop_lds_k(int op, float *o, long ors, t
 {
 	extern __shared__ float lds[];
 	float *lv = lds + lpb * stride; // one value per line (max, then sum or inverse rms)
-	const int bpr = nrow / lpb, r = blockIdx.x / bpr, q0 = (blockIdx.x - r * bpr) * lpb;
-	const int tot = lpb * cols;
+	const int bpr = (nrow + lpb - 1) / lpb, r = blockIdx.x / bpr, q0 = (blockIdx.x - r * bpr) * lpb;
+	const int nl = nrow - q0 < lpb ? nrow - q0 : lpb, tot = nl * cols; // (lines past nl: nothing is loaded, summed or stored)
 	const float *x = a.p + (long)r * a.rs + (long)q0 * cols;
 	// element e of the tile is line e / cols, column e % cols: a thread's
 	// elements e, e + TPB, ... are walked by adding TPB as (dl lines, dc
@@ -361,7 +361,7 @@ __global__ __launch_bounds__(256) void rowop_lds_k(int op, float *o, long ors, t
 			*z = expf(*z - lv[ll]);
 		}
 		__syncthreads();
-		if ((int)threadIdx.x < lpb) lv[threadIdx.x] = line_sum(lds + threadIdx.x * stride, cols);
+		if ((int)threadIdx.x < nl) lv[threadIdx.x] = line_sum(lds + threadIdx.x * stride, cols);
 		__syncthreads();
 		for (int e = threadIdx.x, ll = l0, c = c0; e < tot; e += TPB, step(ll, c)) {
 			float *z = lds + ll * stride + c;
@@ -369,7 +369,7 @@ __global__ __launch_bounds__(256) void rowop_lds_k(int op, float *o, long ors, t
 		}
 	} else {
 		// each square is formed as its value arrives, off the ordered chain of adds
-		if ((int)threadIdx.x < lpb) lv[threadIdx.x] = 1.0f / sqrtf(line_sum<true>(lds + threadIdx.x * stride, cols) / (float)cols + 1e-6f);
+		if ((int)threadIdx.x < nl) lv[threadIdx.x] = 1.0f / sqrtf(line_sum<true>(lds + threadIdx.x * stride, cols) / (float)cols + 1e-6f);
 		__syncthreads();
 		for (int e = threadIdx.x, ll = l0, c = c0; e < tot; e += TPB, step(ll, c)) {
 			float *z = lds + ll * stride + c;
@@ -910,11 +910,13 @@ void tgk_rowop(hipStream_t s, int op, float *o, long ors, tgk_opd a, int nrow, i
 	const int stride = cols % 4 == 0 ? cols + 4 : cols | 1;
 	// LDS: the lines and one value per line (padded to 4)
 	auto lds_bytes = [&](long l) { return (l * stride + ((l + 3) & ~3L)) * 4; };
-	int lpb = 32; // a power of two, so TPB / lpb threads share a line's max
-	while (lpb > 1 && (lds_bytes(lpb) > 65536 || nrow % lpb)) lpb >>= 1;
-	while (lpb > 4 && (long)rows * (nrow / lpb) < 512) lpb >>= 1; // few lines: spread them over more blocks
-	if (cols >= 32 && lpb >= 4 && lds_bytes(lpb) <= 65536 && (long)rows * (nrow / lpb) < (1L << 31))
-		rowop_lds_k<<<(unsigned)(rows * (long)(nrow / lpb)), TPB, (size_t)lds_bytes(lpb), s>>>(op, o, ors, a, nrow, cols, lpb, stride);
+	// a power of two, so TPB / lpb threads of one wave share a line's max; few lines: spread over more blocks. Any number
+	// of lines takes this kernel: 1750 lines of 512 (not a multiple of four) ran one thread a line, 226 us against 11
+	int lpb = 32;
+	while (lpb > 4 && (lds_bytes(lpb) > 65536 || (long)rows * ((nrow + lpb - 1) / lpb) < 512)) lpb >>= 1;
+	const long grid = (long)rows * ((nrow + lpb - 1) / lpb);
+	if (cols >= 32 && lds_bytes(lpb) <= 65536 && grid < (1L << 31))
+		rowop_lds_k<<<(unsigned)grid, TPB, (size_t)lds_bytes(lpb), s>>>(op, o, ors, a, nrow, cols, lpb, stride);
 	else
 		rowop_k<<<blocks_for(total), TPB, 0, s>>>(op, o, ors, a, nrow, cols, total);
 }
