@@ -31,17 +31,21 @@
 #include <hip/hiprtc.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cctype>
 #include <climits>
 #include <cmath>
+#include <condition_variable>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <deque>
 #include <map>
 #include <mutex>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -171,6 +175,112 @@ struct Step {
 	int qv = -1, seg = -1;
 };
 
+// Host threads of one program's host-buffer batches, copying pieces between
+// the caller's pageable buffers and the pinned slots: made at the first copy
+// that is worth sharing, kept between calls (making eight takes 80 us, as
+// long as the copy of a chunk), joined when the program is freed. A worker
+// that finds nothing to do looks again for a while before it sleeps, so that
+// within a batch the next piece does not wait for a wake-up.
+class CopyPool {
+	struct Piece {
+		char *dst;
+		const char *src;
+		size_t n;
+		std::atomic<int> *left;
+	};
+	std::vector<std::thread> th;
+	std::mutex mu;
+	std::condition_variable cv;
+	std::deque<Piece> q;
+	std::atomic<int> queued{ 0 };
+	bool stop = false, started = false;
+
+	bool pop(Piece &x)
+	{
+		std::lock_guard<std::mutex> lk(mu);
+		if (q.empty()) return false;
+		x = q.front();
+		q.pop_front();
+		queued.fetch_sub(1, std::memory_order_relaxed);
+		return true;
+	}
+	static void run(const Piece &x)
+	{
+		memcpy(x.dst, x.src, x.n);
+		x.left->fetch_sub(1, std::memory_order_release);
+	}
+	void start()
+	{
+		if (started) return;
+		started = true;
+		const unsigned hc = std::thread::hardware_concurrency();
+		for (unsigned i = 0; i < std::min(11u, hc > 1 ? hc - 1 : 0u); i++) {
+			try {
+				th.emplace_back([this] { work(); });
+			} catch (const std::system_error &) {
+				break; // the threads there are, and the caller, do it
+			}
+		}
+	}
+	void work()
+	{
+		for (;;) {
+			Piece x;
+			for (int i = 0; i < 2000 && !queued.load(std::memory_order_relaxed); i++) std::this_thread::yield();
+			if (pop(x)) {
+				run(x);
+				continue;
+			}
+			std::unique_lock<std::mutex> lk(mu);
+			cv.wait(lk, [&] { return stop || !q.empty(); });
+			if (stop) return;
+		}
+	}
+
+public:
+	// pieces of a copy: out, whole huge pages of the caller's buffer (a fresh one's first writes map it; two threads
+	// that meet in one page both clear it)
+	static constexpr size_t IN_PIECE = (size_t)512 << 10, OUT_PIECE = (size_t)2 << 20;
+	// queue a copy in pieces; `left` counts its pieces down (it, dst and src outlive them: wait() before they go)
+	void submit(void *dst, const void *src, size_t n, size_t piece, std::atomic<int> &left)
+	{
+		if (n < (size_t)1 << 20) { // not worth a wake-up
+			memcpy(dst, src, n);
+			return;
+		}
+		start();
+		{
+			std::lock_guard<std::mutex> lk(mu);
+			for (size_t a = 0; a < n;) {
+				const size_t m = std::min(n - a, piece - ((uintptr_t)dst + a) % piece);
+				left.fetch_add(1, std::memory_order_relaxed);
+				q.push_back({ (char *)dst + a, (const char *)src + a, m, &left });
+				queued.fetch_add(1, std::memory_order_relaxed);
+				a += m;
+			}
+		}
+		cv.notify_all();
+	}
+	// until the copies that `left` counts are done, helping
+	void wait(std::atomic<int> &left)
+	{
+		Piece x;
+		while (left.load(std::memory_order_acquire) > 0) {
+			if (pop(x)) run(x);
+			else std::this_thread::yield();
+		}
+	}
+	~CopyPool()
+	{
+		{
+			std::lock_guard<std::mutex> lk(mu);
+			stop = true;
+		}
+		cv.notify_all();
+		for (auto &t : th) t.join();
+	}
+};
+
 } // namespace
 
 struct tg_hip_prog {
@@ -215,8 +325,9 @@ struct tg_hip_prog {
 	hipModule_t rp_mod = nullptr;  // the row program compiled for this model
 	hipFunction_t rp_fn = nullptr; // its kernel (null: the interpreter runs the program)
 	std::string rp_why;            // why the program runs in the interpreter
-	// host-buffer batches: a three-slot pipeline (pinned staging, device buffers, copy streams, events)
-	static constexpr int NSL = 3; // pipeline slots
+	// host-buffer batches: a pipeline of slots (pinned staging, device buffers, copy streams, events)
+	static constexpr int NSL = 4;
+	CopyPool copies;
 	struct HostPipe {
 		long chunk = 0;                                            // rows per chunk
 		void *h_in[NSL] = {}, *h_out[NSL] = {};                    // pinned staging
@@ -2433,24 +2544,6 @@ void destroy(tg_hip_prog *p)
 	delete p;
 }
 
-// memcpy on a few host threads (pageable caller memory <-> pinned staging)
-void par_copy(void *dst, const void *src, size_t n)
-{
-	const size_t piece = (size_t)4 << 20;
-	const int nt = n < 2 * piece ? 1 : (int)std::min<size_t>(8, n / piece);
-	if (nt == 1) {
-		memcpy(dst, src, n);
-		return;
-	}
-	std::vector<std::thread> th;
-	const size_t per = (n + nt - 1) / nt;
-	for (int t = 0; t < nt; t++) {
-		const size_t a = (size_t)t * per, b = std::min(n, a + per);
-		if (a < b) th.emplace_back([=] { memcpy((char *)dst + a, (const char *)src + a, b - a); });
-	}
-	for (auto &x : th) x.join();
-}
-
 // Pinned host allocations made by tg_hip_host_alloc: start -> size. A row or
 // output buffer inside one moves over PCIe directly (no staging copy).
 std::mutex g_pinned_mu;
@@ -2472,8 +2565,9 @@ bool host_pipe_init(tg_hip_prog *p)
 	auto &h = p->hp;
 	if (h.chunk) return true;
 	const long per = p->m->per, nout = p->m->nout, nt = p->m->nthink ? p->m->nthink : 1;
-	// about 16 MiB of rows per chunk: copies of one chunk overlap the compute of the next
-	long c = (16l << 20) / (4 * (per > nout ? per : nout));
+	// up to 8 MiB of rows per chunk: smaller ones travel as well (4 MiB: 51 GB/s, 16 MiB: 56) but compute less well
+	// (2048 rows of a 512-2048-2048-512 MLP 180 us, 4096 of them 200)
+	long c = (8l << 20) / (4 * (per > nout ? per : nout));
 	c = c < 256 ? 256 : c;
 	h.chunk = c < p->max_rows ? c : p->max_rows;
 	bool ok = hipok(hipStreamCreate(&h.h2d), "stream") && hipok(hipStreamCreate(&h.d2h), "stream");
@@ -2493,14 +2587,19 @@ bool host_pipe_init(tg_hip_prog *p)
 }
 
 // Host buffers, the block loop of `tgc batch`: rows go in chunks through a
-// three-slot pipeline. Chunk i uses slot i % 3: its rows are copied into the
-// slot's pinned buffer on the host, up to the device on the copy-in stream,
-// computed on the program's stream, and down on the copy-out stream; each
-// stream waits for the event of the step before it, and a slot is refilled
-// only after its previous chunk has left it. So chunk i + 1 travels while
-// chunk i computes. Passes run in input order on one stream, as before.
+// pipeline of NSL slots. Chunk i uses slot i % NSL: its rows are copied into
+// the slot's pinned buffer on the host, up to the device on the copy-in
+// stream, computed on the program's stream, and down on the copy-out stream;
+// each stream waits for the event of the step before it. A chunk whose
+// outputs have arrived is copied out by the pool's threads while the caller's
+// thread brings in the next, and a slot is refilled only after its previous
+// chunk has left it. Passes run in input order on one stream, as before.
 // Rows, outputs or steps in memory from tg_hip_host_alloc skip the host
-// copies: the transfers read and write the caller's buffers directly.
+// copies: the transfers read and write the caller's buffers directly. A call
+// of one chunk has nothing to overlap and goes down one stream, without the
+// events between three. 8192 rows of 512 values in and out, pageable, through a
+// 512-2048-2048-512 MLP: 1.41-1.51 ms in one chunk and three slots,
+// 0.9-1.1 now; 3000 rows 0.91 ms down three streams, 0.56 down one.
 int batch_host(tg_hip_prog *p, const void *rows, long nrows, void *out, int *steps)
 {
 	if (!p) {
@@ -2508,55 +2607,80 @@ int batch_host(tg_hip_prog *p, const void *rows, long nrows, void *out, int *ste
 		return -1;
 	}
 	if (!host_pipe_init(p)) return -1;
+	constexpr int NSL = tg_hip_prog::NSL;
 	auto &h = p->hp;
 	const long per = p->m->per, nout = p->m->nout, nt = p->m->nthink ? p->m->nthink : 1;
 	const bool din = in_pinned(rows, (size_t)nrows * per * 4), dout = in_pinned(out, (size_t)nrows * nout * 4);
 	const bool dsteps = steps && in_pinned(steps, (size_t)nrows * nt * 4);
-	// chunks of about 16 MiB of rows through the staging slots (the host copies
-	// want large pieces); a quarter of that when nothing is staged, so the
-	// first chunk's upload and the last one's download, which nothing
-	// overlaps, are short
-	const long C = din && dout ? std::max(64L, h.chunk / 4) : h.chunk;
-	const long nch = (nrows + C - 1) / C;
+	// equal chunks of at most h.chunk rows, half that for what nothing stages, so that what nothing overlaps (the first
+	// one's way in, the last one's way out) is short
+	const long cmax = din && dout ? std::max(64L, (h.chunk + 1) / 2) : h.chunk;
+	const long nch0 = (nrows + cmax - 1) / cmax, C = nch0 > 1 ? (nrows + nch0 - 1) / nch0 : cmax, nch = (nrows + C - 1) / C;
+	const hipStream_t up = nch > 1 ? h.h2d : p->st, down = nch > 1 ? h.d2h : p->st;
 	float ms_total = 0;
-	auto finish = [&](long i) -> bool { // chunk i's outputs to the caller
-		const int k = (int)(i % tg_hip_prog::NSL);
-		const long r0 = i * C, cnt = nrows - r0 < C ? nrows - r0 : C;
-		if (!hipok(hipEventSynchronize(h.down[k]), "outputs to host")) return false;
-		if (!dout) par_copy((char *)out + (size_t)r0 * nout * 4, h.h_out[k], (size_t)cnt * nout * 4);
+	struct Left { // pieces of each slot's copies; none outlives the call, whatever it returns
+		CopyPool &pool;
+		std::atomic<int> in{ 0 }, out[NSL];
+		Left(CopyPool &c) : pool(c)
+		{
+			for (auto &x : out) x = 0;
+		}
+		~Left()
+		{
+			pool.wait(in);
+			for (auto &x : out) pool.wait(x);
+		}
+	} left(p->copies);
+	long arrived = 0; // chunks before it are down, their copies to the caller begun
+	auto arrive = [&](bool wait) -> bool { // the next chunk's outputs, if they are down (or once they are)
+		const long i = arrived, r0 = i * C, cnt = nrows - r0 < C ? nrows - r0 : C;
+		const int k = (int)(i % NSL);
+		const hipError_t e = wait ? hipEventSynchronize(h.down[k]) : hipEventQuery(h.down[k]);
+		if (e == hipErrorNotReady) return true;
+		if (!hipok(e, "outputs to host")) return false;
+		if (!dout) p->copies.submit((char *)out + (size_t)r0 * nout * 4, h.h_out[k], (size_t)cnt * nout * 4, CopyPool::OUT_PIECE, left.out[k]);
 		if (steps && p->m->nthink && !dsteps) memcpy(steps + (size_t)r0 * nt, h.h_steps[k], (size_t)cnt * nt * 4);
 		float ms = 0;
 		(void)hipEventElapsedTime(&ms, h.t0[k], h.t1[k]);
 		ms_total += ms;
+		arrived++;
 		return true;
 	};
 	for (long i = 0; i < nch; i++) {
-		const int k = (int)(i % tg_hip_prog::NSL);
+		const int k = (int)(i % NSL);
 		const long r0 = i * C, cnt = nrows - r0 < C ? nrows - r0 : C;
-		if (i >= tg_hip_prog::NSL && !finish(i - tg_hip_prog::NSL)) return -1; // the slot's previous chunk is out: its buffers are free
+		if (i >= NSL) { // the slot's previous chunk is out: its buffers are free
+			if (arrived <= i - NSL && !arrive(true)) return -1;
+			p->copies.wait(left.out[k]);
+		}
 		const void *src = (const char *)rows + (size_t)r0 * per * 4;
 		if (!din) {
-			par_copy(h.h_in[k], src, (size_t)cnt * per * 4);
+			p->copies.submit(h.h_in[k], src, (size_t)cnt * per * 4, CopyPool::IN_PIECE, left.in);
+			p->copies.wait(left.in);
 			src = h.h_in[k];
 		}
-		if (!hipok(hipMemcpyAsync(h.d_in[k], src, (size_t)cnt * per * 4, hipMemcpyHostToDevice, h.h2d), "rows to device") ||
-		    !hipok(hipEventRecord(h.up[k], h.h2d), "event") || !hipok(hipStreamWaitEvent(p->st, h.up[k], 0), "wait"))
-			return -1;
+		if (!hipok(hipMemcpyAsync(h.d_in[k], src, (size_t)cnt * per * 4, hipMemcpyHostToDevice, up), "rows to device")) return -1;
+		if (nch > 1 && (!hipok(hipEventRecord(h.up[k], up), "event") || !hipok(hipStreamWaitEvent(p->st, h.up[k], 0), "wait"))) return -1;
 		(void)hipEventRecord(h.t0[k], p->st);
 		if (run_pass(p, h.d_in[k], (int)cnt, h.d_out[k], h.d_steps[k])) return -1;
 		(void)hipEventRecord(h.t1[k], p->st);
 		void *odst = dout ? (void *)((char *)out + (size_t)r0 * nout * 4) : h.h_out[k];
 		void *sdst = dsteps ? (void *)(steps + (size_t)r0 * nt) : (void *)h.h_steps[k];
-		if (!hipok(hipEventRecord(h.done[k], p->st), "event") || !hipok(hipStreamWaitEvent(h.d2h, h.done[k], 0), "wait") ||
-		    !hipok(hipMemcpyAsync(odst, h.d_out[k], (size_t)cnt * nout * 4, hipMemcpyDeviceToHost, h.d2h), "outputs to host"))
-			return -1;
+		if (nch > 1 && (!hipok(hipEventRecord(h.done[k], p->st), "event") || !hipok(hipStreamWaitEvent(down, h.done[k], 0), "wait"))) return -1;
+		if (!hipok(hipMemcpyAsync(odst, h.d_out[k], (size_t)cnt * nout * 4, hipMemcpyDeviceToHost, down), "outputs to host")) return -1;
 		if (steps && p->m->nthink &&
-		    !hipok(hipMemcpyAsync(sdst, h.d_steps[k], (size_t)cnt * nt * 4, hipMemcpyDeviceToHost, h.d2h), "steps to host"))
+		    !hipok(hipMemcpyAsync(sdst, h.d_steps[k], (size_t)cnt * nt * 4, hipMemcpyDeviceToHost, down), "steps to host"))
 			return -1;
-		if (!hipok(hipEventRecord(h.down[k], h.d2h), "event")) return -1;
+		if (!hipok(hipEventRecord(h.down[k], down), "event")) return -1;
+		while (arrived < i) { // what came down meanwhile
+			const long a = arrived;
+			if (!arrive(false)) return -1;
+			if (arrived == a) break;
+		}
 	}
-	for (long i = nch > tg_hip_prog::NSL ? nch - tg_hip_prog::NSL : 0; i < nch; i++)
-		if (!finish(i)) return -1;
+	while (arrived < nch)
+		if (!arrive(true)) return -1;
+	for (auto &x : left.out) p->copies.wait(x);
 	collect_timing(p);
 	if (steps && !p->m->nthink) memset(steps, 0, (size_t)nrows * sizeof *steps); /* no think loop: one zero slot per row */
 	p->stats.rows = (int)nrows;

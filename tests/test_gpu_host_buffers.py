@@ -64,3 +64,22 @@ def test_host_free_refuses_foreign_pointers():
     hb = hip.HostBuffer(64)
     assert hip.lib().tg_hip_host_free(hb.ptr + 16) == -1  # inside, but not the start
     hb.free()
+
+
+def test_pageable_rows_in_one_chunk_and_many():
+    """One, two and several chunks of staged rows, slots refilled, shared
+    copies and whole ones: the bits of the same rows on device buffers."""
+    W = synth.rand(1, 0.05, 96 * 64).reshape(96, 64)
+    text = synth.linear_tgir("chunks", W, 8)
+    n = 150001  # 8 MiB chunks of 21845 rows of outputs: seven, the slots used twice
+    x = synth.rand(3, 1.0, n * 64).reshape(n, 64)
+    prog = hip.Program(text, max_rows=n)
+    dx, dy = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer(n * 96 * 4)
+    prog.batch_device(dx.ptr, n, dy.ptr)
+    prog.sync()
+    want = dy.to_array(np.float32, (n, 96))
+    for rows in (1, 21845, 21846, n):
+        print("case host chunks", rows, flush=True)
+        got, steps = prog.batch(x[:rows])
+        assert np.array_equal(got.view(np.uint32), want[:rows].view(np.uint32)) and not steps.any()
+    prog.close()
