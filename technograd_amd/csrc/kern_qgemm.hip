@@ -112,20 +112,40 @@ __device__ inline long long wave_sum(long long v)
 	return v;
 }
 
-// inputs k0 .. k0 + 15 of a row. The addresses are clamped into the row
+// 16 bytes of a row that starts at any float
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// v holds the row's last 16 inputs (K - 16 ..) where it should hold inputs
+// k0 .. k0 + 15, k0 < K < k0 + 16: moved down by k0 - (K - 16), zeros from K on
+// (four conditional moves of the whole group; other lanes' groups are left)
+__device__ inline void tail16(float *v, int k0, int K)
+{
+	const int sh = k0 < K && k0 + 16 > K ? k0 + 16 - K : 0;
+#pragma unroll
+	for (int b = 8; b > 0; b >>= 1)
+#pragma unroll
+		for (int i = 0; i < 16; i++) v[i] = sh & b ? (i + b < 16 ? v[i + b] : 0.0f) : v[i];
+}
+
+// Inputs k0 .. k0 + 15 of a row. The addresses are clamped into the row
 // instead of branched on, so the loads of several calls can all be in flight
-// before the first value is used. vec (unit stride, 16-byte aligned row, K a
-// multiple of 16, so whole float4s): a group at or past K reads the row's
-// first 16 inputs instead, which leave the row's max and NaN flag unchanged;
-// the caller writes such a group as zero digits (tgq_put16's `zero`).
-// Otherwise inputs at and beyond K read as zeros.
+// before the first value is used. VEC (unit stride, K >= 16): 16-byte loads
+// at any alignment of the row (its groups are 64 bytes apart, so what a load
+// straddles the next one reads as well); the group that ends past K loads
+// the row's last 16 inputs, and fix16 moves them into place, zeros past K,
+// once every load of the caller's has been issued; a group
+// at or past K reads the row's first 16 inputs, which leave the row's max
+// and NaN flag unchanged: the caller writes it as zero digits (tgq_put16's
+// `zero`). With a load per input the digits of 700 rows of 2917 were 30 us of
+// a product's 56; it takes 42 so. Otherwise (strided rows, short ones) inputs at and beyond K read as
+// zeros, one load each.
 template <bool VEC>
 __device__ inline void load16(float *v, const float *x, long xk, int k0, int K)
 {
 	if (VEC) {
-		const float *p = x + (k0 < K ? k0 : 0);
+		const float *p = x + (k0 < K ? (k0 + 16 <= K ? k0 : K - 16) : 0);
 		for (int i = 0; i < 4; i++) {
-			const float4 f = *(const float4 *)(p + 4 * i);
+			const f4u f = *(const f4u *)(p + 4 * i);
 			v[4 * i] = f.x, v[4 * i + 1] = f.y, v[4 * i + 2] = f.z, v[4 * i + 3] = f.w;
 		}
 	} else {
@@ -136,6 +156,12 @@ __device__ inline void load16(float *v, const float *x, long xk, int k0, int K)
 		}
 	}
 }
+template <bool VEC>
+__device__ inline void fix16(float *v, int k0, int K)
+{
+	if (VEC && (K & 15) && __any(k0 < K && k0 + 16 > K)) tail16(v, k0, K); // (the wave that holds the row's end)
+}
+inline bool row_vec(const tgk_qgemm_args *a) { return a->xk == 1 && a->w->K >= 16; }
 
 // One wave per activation row (4 rows per block): exponent, digits, sum of q,
 // special flag. Lane l owns inputs 1024 s + 16 l .. +15 of each 1024-input
@@ -149,7 +175,7 @@ __global__ __launch_bounds__(256) void digits_k(tgk_qgemm_args a, Scratch s, int
 	if (m >= M) return; // the whole wave leaves; the kernel has no block barrier
 	const float *x = xrow(a, m);
 	const long xk = a.xk;
-	const bool vec = xk == 1 && ((size_t)x & 15) == 0 && (K & 15) == 0;
+	const bool vec = xk == 1 && K >= 16;
 	const int nsl = (Kp + 1023) / 1024;
 	float v[SL][16];
 	unsigned mb = 0; // max |x| as bits (tgq_scan16)
@@ -160,6 +186,8 @@ __global__ __launch_bounds__(256) void digits_k(tgk_qgemm_args a, Scratch s, int
 			for (int t = 0; t < SL; t++) load16<true>(v[t], x, xk, (t0 + t) * 1024 + lane * 16, K);
 		else
 			for (int t = 0; t < SL; t++) load16<false>(v[t], x, xk, (t0 + t) * 1024 + lane * 16, K);
+		if (vec)
+			for (int t = 0; t < SL; t++) fix16<true>(v[t], (t0 + t) * 1024 + lane * 16, K);
 	};
 	for (int t0 = 0; t0 < nsl; t0 += SL) {
 		fetch(t0);
@@ -205,7 +233,7 @@ __global__ __launch_bounds__(256) void digits_k(tgk_qgemm_args a, Scratch s, int
 		auto ld = [&](int g, float *v) {
 			if (g * 16 >= K)
 				for (int i = 0; i < 16; i++) v[i] = 0.0f;
-			else if (vec) load16<true>(v, x, xk, g * 16, K);
+			else if (vec) load16<true>(v, x, xk, g * 16, K), fix16<true>(v, g * 16, K);
 			else load16<false>(v, x, xk, g * 16, K);
 		};
 		tgq_resolve_row(&hist[threadIdx.x >> 6], ld, K, Kp, E, blk, &s.qsum[m], &s.e[m], &s.special[m], s.ok + (long)m * nout,
@@ -240,6 +268,10 @@ __global__ __launch_bounds__(1024) void digits_tile16_k(tgk_qgemm_args a, Scratc
 	for (int j = 0; j < NKB; j++) {
 		const int kb = 2 * (w + j * W) + par;
 		load16<VEC>(v[j], x, a.xk, kb < nkb ? kb * 32 + half * 16 : K, K); // past the row: zeros
+	}
+	for (int j = 0; j < NKB; j++) {
+		const int kb = 2 * (w + j * W) + par;
+		fix16<VEC>(v[j], kb < nkb ? kb * 32 + half * 16 : K, K);
 		tgq_scan16(v[j], mb);
 	}
 	float mx;
@@ -303,7 +335,7 @@ __global__ __launch_bounds__(1024) void digits_tile16_k(tgk_qgemm_args a, Scratc
 			auto ld = [&](int g, float *v) {
 				if (g * 16 >= K)
 					for (int i = 0; i < 16; i++) v[i] = 0.0f;
-				else load16<VEC>(v, xr, a.xk, g * 16, K);
+				else load16<VEC>(v, xr, a.xk, g * 16, K), fix16<VEC>(v, g * 16, K);
 			};
 			tgq_resolve_row(&hist[w], ld, K, Kp, sE[r], tgq_row_base(s.dig, m, Kp), &s.qsum[m], &s.e[m], &s.special[m], s.ok + (long)m * nout,
 					s.ox + (long)m * nout, nout, lane);
@@ -328,6 +360,10 @@ __device__ inline void row_digits(const tgk_qgemm_args &a, const Scratch &s, int
 	for (int g = 0; g < G; g++) {
 		const int j = tid + g * NT;
 		load16<VEC>(v[g], x, a.xk, j < ng ? j * 16 : K, K); // past the row: zeros
+	}
+	for (int g = 0; g < G; g++) {
+		const int j = tid + g * NT;
+		fix16<VEC>(v[g], j < ng ? j * 16 : K, K);
 		tgq_scan16(v[g], mb);
 	}
 	float mx;
@@ -379,7 +415,7 @@ __device__ inline void row_digits(const tgk_qgemm_args &a, const Scratch &s, int
 		auto ld = [&](int g, float *v) {
 			if (g * 16 >= K)
 				for (int i = 0; i < 16; i++) v[i] = 0.0f;
-			else load16<VEC>(v, x, a.xk, g * 16, K);
+			else load16<VEC>(v, x, a.xk, g * 16, K), fix16<VEC>(v, g * 16, K);
 		};
 		tgq_resolve_row(&hist, ld, K, Kp, E, blk, &s.qsum[m], &s.e[m], &s.special[m], s.ok + (long)m * nout, s.ox + (long)m * nout, nout,
 				lane);
@@ -414,7 +450,7 @@ __global__ __launch_bounds__(256) void resolve_k(tgk_qgemm_args a, Scratch s, in
 			auto ld = [&](int g, float *v) {
 				if (g * 16 >= K)
 					for (int i = 0; i < 16; i++) v[i] = 0.0f;
-				else load16<VEC>(v, x, a.xk, g * 16, K);
+				else load16<VEC>(v, x, a.xk, g * 16, K), fix16<VEC>(v, g * 16, K);
 			};
 			tgq_resolve_row(&hist[wave], ld, K, Kp, s.e[m], tgq_row_base(s.dig, (int)m, Kp), &s.qsum[m], &s.e[m], &s.special[m],
 					s.ok + m * nout, s.ox + m * nout, nout, lane);
@@ -1537,14 +1573,14 @@ __device__ int fused_resolve(const tgk_qweight &w, const Scratch &s, const float
 // [block][digit][half][16 bytes], read by every lane with the same block and
 // half (a broadcast).
 // FUSED: the workgroup makes those digits itself from the row (unit stride,
-// 16-byte aligned, K a multiple of 16): max |x|, exponent, peak test and sum
+// any alignment; TAIL: K not a multiple of 16, the last group as in load16): max |x|, exponent, peak test and sum
 // of q by block reductions, exactly as the digit kernels do, so no digit
 // kernel runs before it; workgroup 0 also writes the digits and row data to
 // the scratch (a later product may reuse them). Otherwise the digits come
 // from the scratch. The row and digit loads are issued before the weight
 // loads and waited for with a count that leaves the weights in flight (loads
 // complete in order), all as inline assembly like qgemv_k's.
-template <int NL, bool FUSED>
+template <int NL, bool FUSED, bool TAIL = false>
 __global__ __launch_bounds__(256) void gemv1_k(tgk_qgemm_args a, tgk_qweight w, Scratch s)
 {
 	constexpr int GX = 2; // 16-input groups of the row per thread (FUSED: K <= 8192)
@@ -1562,7 +1598,7 @@ __global__ __launch_bounds__(256) void gemv1_k(tgk_qgemm_args a, tgk_qweight w, 
 	const uint8_t *xb = sgpr_ptr((const uint8_t *)xrow(a, 0));
 	if constexpr (FUSED) {
 		for (int u = 0; u < GX; u++) {
-			const int k0 = 16 * (tid + 256 * u), kk = k0 < K ? k0 : 0; // past the row: its first group (not used)
+			const int k0 = 16 * (tid + 256 * u), kk = k0 < K ? (TAIL && k0 + 16 > K ? K - 16 : k0) : 0; // past the row: its first group (not used)
 			for (int i = 0; i < 4; i++) ld16(xv[u * 4 + i], xb, (unsigned)(kk + 4 * i) * 4);
 		}
 	} else {
@@ -1591,6 +1627,7 @@ __global__ __launch_bounds__(256) void gemv1_k(tgk_qgemm_args a, tgk_qweight w, 
 		for (int u = 0; u < GX; u++) {
 			for (int i = 0; i < 4; i++)
 				for (int e = 0; e < 4; e++) v[u][4 * i + e] = __int_as_float(xv[u * 4 + i][e]);
+			if constexpr (TAIL) tail16(v[u], 16 * (tid + 256 * u), K);
 			if (16 * (tid + 256 * u) < K) tgq_scan16(v[u], mb);
 		}
 		float mx;
@@ -1712,11 +1749,16 @@ bool launch_gemv1(hipStream_t st, const tgk_qgemm_args *a, Scratch s)
 	const tgk_qweight *w = a->w;
 	const int kblocks = w->Kp / 32, g = w->Cp / 16;
 	if (a->M != 1 || w->bits != 4 || kblocks > 256) return false;
-	if (kblocks <= 16) gemv1_k<1, FUSED><<<g, 256, 0, st>>>(*a, *w, s);
-	else if (kblocks <= 32) gemv1_k<2, FUSED><<<g, 256, 0, st>>>(*a, *w, s);
-	else if (kblocks <= 64) gemv1_k<4, FUSED><<<g, 256, 0, st>>>(*a, *w, s);
-	else if (kblocks <= 128) gemv1_k<8, FUSED><<<g, 256, 0, st>>>(*a, *w, s);
-	else gemv1_k<16, FUSED><<<g, 256, 0, st>>>(*a, *w, s);
+	auto run = [&](auto tail) {
+		constexpr bool T = FUSED && decltype(tail)::value;
+		if (kblocks <= 16) gemv1_k<1, FUSED, T><<<g, 256, 0, st>>>(*a, *w, s);
+		else if (kblocks <= 32) gemv1_k<2, FUSED, T><<<g, 256, 0, st>>>(*a, *w, s);
+		else if (kblocks <= 64) gemv1_k<4, FUSED, T><<<g, 256, 0, st>>>(*a, *w, s);
+		else if (kblocks <= 128) gemv1_k<8, FUSED, T><<<g, 256, 0, st>>>(*a, *w, s);
+		else gemv1_k<16, FUSED, T><<<g, 256, 0, st>>>(*a, *w, s);
+	};
+	if (w->K & 15) run(std::true_type{});
+	else run(std::false_type{});
 	return true;
 }
 
@@ -2071,8 +2113,7 @@ void tgk_qgemm_digits(hipStream_t st, const tgk_qgemm_args *a, void *scratch)
 	const Scratch s = carve(scratch, Mp, w->Kp);
 	const int nkb = w->Kp / 32, M = a->M, K = w->K;
 	if (M >= 512 && nkb <= 128) { // 16 rows per block
-		const bool vec = a->xk == 1 && ((size_t)a->x & 15) == 0 && (a->xr & 3) == 0 && (a->ni == 1 || (a->xj & 3) == 0) &&
-				 (K & 15) == 0;
+		const bool vec = row_vec(a);
 		// 16 waves; 8 for many rows of at most 2048 inputs: then two blocks fit
 		// on a CU (registers), one loading while the other computes and stores
 		// (measured: K = 2048, 65536 rows: 178 us against 235 with one 32-row
@@ -2102,8 +2143,7 @@ void tgk_qgemm_digits(hipStream_t st, const tgk_qgemm_args *a, void *scratch)
 		}
 		if (defer) tgk_qgemm_split(st, a, scratch);
 	} else if (M < 512 && w->Kp >= 2048 && w->Kp <= 16384) { // few long rows: a block per row
-		const bool vec = a->xk == 1 && ((size_t)a->x & 15) == 0 && (a->xr & 3) == 0 && (a->ni == 1 || (a->xj & 3) == 0) &&
-				 (K & 15) == 0;
+		const bool vec = row_vec(a);
 		const int G = (w->Kp / 16 + 255) / 256;
 		if (G <= 1) {
 			if (vec) digits_row_k<1, true><<<M, 256, 0, st>>>(*a, s, K, w->Kp, M);
@@ -2129,7 +2169,7 @@ void tgk_qgemm_split(hipStream_t st, const tgk_qgemm_args *a, void *scratch)
 	const Scratch s = carve(scratch, (int)round_up(M, BM), w->Kp);
 	const long blocks = (M + 3) / 4;
 	const unsigned nb = (unsigned)(blocks < 16384 ? blocks : 16384);
-	const bool vec = a->xk == 1 && ((size_t)a->x & 15) == 0 && (a->xr & 3) == 0 && (a->ni == 1 || (a->xj & 3) == 0) && (w->K & 15) == 0;
+	const bool vec = row_vec(a);
 	if (vec) resolve_k<true><<<nb, 256, 0, st>>>(*a, s, w->K, w->Kp, M);
 	else resolve_k<false><<<nb, 256, 0, st>>>(*a, s, w->K, w->Kp, M);
 }
@@ -2168,8 +2208,7 @@ void tgk_qgemm_chain(hipStream_t st, const tgk_qgemm_args *a)
 bool tgk_qgemm_fusable(const tgk_qgemm_args *a)
 {
 	const tgk_qweight *w = a->w;
-	return w && w->w && a->x && a->M == 1 && w->bits == 4 && w->K > TGK_REFLOOP_K && w->Kp <= 8192 && a->xk == 1 &&
-	       ((size_t)a->x & 15) == 0 && (w->K & 15) == 0;
+	return w && w->w && a->x && a->M == 1 && w->bits == 4 && w->K > TGK_REFLOOP_K && w->Kp <= 8192 && a->xk == 1;
 }
 
 int tgk_qgemm_fused(hipStream_t st, const tgk_qgemm_args *a, void *scratch)

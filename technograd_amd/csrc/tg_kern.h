@@ -305,8 +305,8 @@ typedef struct {
  * tgk_qgemm_split launch nothing for them) */
 #define TGK_REFLOOP_K 32
 /* scratch: bytes needed for M rows of K inputs */
-/* One row of int4 weights (M = 1, unit-stride 16-byte-aligned row, K a
- * multiple of 16, K <= 8192): tgk_qgemm_fused computes the digits inside
+/* One row of int4 weights (M = 1, unit stride, TGK_REFLOOP_K < K <= 8192):
+ * tgk_qgemm_fused computes the digits inside
  * the product's own kernel (and leaves them in the scratch like
  * tgk_qgemm_digits); other cases fall back to digits + product. */
 bool tgk_qgemm_fusable(const tgk_qgemm_args *a);
