@@ -188,6 +188,32 @@ __device__ inline long long tgq_put16(int8_t *blk, int k0, const float *v, int E
 	return qs;
 }
 
+// ---- a wave's sums ----
+
+// v of the lanes summed (or their unsigned max), in every lane: data-parallel
+// moves, a few cycles a step where a __shfl is a round trip through LDS
+template <int CTRL, int ROWS> __device__ inline int tgq_dpp(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false); }
+__device__ inline int tgq_wave_add(int v)
+{
+	v += tgq_dpp<0x111, 0xf>(v); // row_shr 1, 2, 4, 8: lane 15 of a row of 16 holds the row's sum
+	v += tgq_dpp<0x112, 0xf>(v);
+	v += tgq_dpp<0x114, 0xf>(v);
+	v += tgq_dpp<0x118, 0xf>(v);
+	v += tgq_dpp<0x142, 0xa>(v); // row_bcast 15 into rows 1 and 3, row_bcast 31 into rows 2 and 3
+	v += tgq_dpp<0x143, 0xc>(v);
+	return __builtin_amdgcn_readlane(v, 63);
+}
+__device__ inline unsigned tgq_wave_umax(unsigned v)
+{
+	v = max(v, (unsigned)tgq_dpp<0x111, 0xf>((int)v));
+	v = max(v, (unsigned)tgq_dpp<0x112, 0xf>((int)v));
+	v = max(v, (unsigned)tgq_dpp<0x114, 0xf>((int)v));
+	v = max(v, (unsigned)tgq_dpp<0x118, 0xf>((int)v));
+	v = max(v, (unsigned)tgq_dpp<0x142, 0xa>((int)v));
+	v = max(v, (unsigned)tgq_dpp<0x143, 0xc>((int)v));
+	return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 // ---- resolving a candidate row (a whole wave) ----
 
 __device__ inline int tgq_wave_sum(int v)
@@ -350,6 +376,58 @@ __device__ inline TgqCoarse tgq_coarse_wave_sum(TgqCoarse c)
 	return c;
 }
 
+// What tgq_put16 and tgq_coarse16 add up, of a row's inputs in a wave's hands:
+// sum of q, candidate tally, coarse groups. The same in every lane.
+struct TgqRowSums {
+	long long qs, tl;
+	TgqCoarse co;
+};
+
+// Digits of four inputs a lane (k0 .. k0 + 3 of the row at blk, k0 a multiple
+// of 4; zeros at and past the row's end, stored where `in`), and their sums
+// over the wave: a row of 1024 inputs is four waves' work of a quad a lane,
+// where 16 inputs a lane are one wave's, four times as long. |q| <= 8355328,
+// so 256 of them sum within 32 bits. Whole waves only; `special` (the row's)
+// is the same in all lanes.
+__device__ inline void tgq_quad(int8_t *blk, int k0, bool in, const float *v, int E, int special, TgqRowSums &s)
+{
+	unsigned w0 = 0, w1 = 0, w2 = 0;
+	if (!special) {
+		int qs = 0, nx = 0, n0 = 0, n1 = 0, nz = 0;
+		unsigned aq = 0, a0 = 0, a1 = 0, u[4];
+#pragma unroll
+		for (int i = 0; i < 4; i++) {
+			const float sv = ldexpf(v[i], 23 - E), rq = rintf(sv);
+			const int q = (int)rq;
+			const unsigned m = (unsigned)abs(q);
+			const bool g0 = m >= (1u << 22), g1 = !g0 && m >= (1u << 21);
+			qs += q;
+			aq += m;
+			a0 += g0 ? m : 0u, a1 += g1 ? m : 0u;
+			nx += __popcll(__ballot(rq != sv)), nz += __popcll(__ballot(v[i] != 0.0f));
+			n0 += __popcll(__ballot(g0)), n1 += __popcll(__ballot(g1));
+			u[i] = (unsigned)(q + 0x808080);
+		}
+		tgq_pack4(u, w0, w1, w2);
+		s.qs += tgq_wave_add(qs);
+		s.tl += (long long)(unsigned)tgq_wave_add((int)aq) + ((long long)nx << TGQ_TALLY_SHIFT);
+		s.co.cnt += (unsigned long long)n0 + ((unsigned long long)n1 << 21) + ((unsigned long long)nz << 42);
+		s.co.s0 += (unsigned)tgq_wave_add((int)a0), s.co.s1 += (unsigned)tgq_wave_add((int)a1);
+	}
+	if (in) {
+		int8_t *p = blk + (k0 >> 5) * 3072 + ((k0 >> 4) & 1) * 512 + (k0 & 15);
+		*(unsigned *)p = w0;
+		*(unsigned *)(p + 1024) = w1;
+		*(unsigned *)(p + 2048) = w2;
+	}
+}
+
+// the running max of |x| over four inputs, as tgq_scan16 keeps it
+__device__ inline void tgq_scan4(const float *v, unsigned &mb)
+{
+	for (int i = 0; i < 4; i++) mb = max(mb, __float_as_uint(v[i]) & 0x7fffffffu);
+}
+
 // whether a candidate row with the tally `tally` keeps its grid by the coarse test alone
 __device__ inline bool tgq_coarse_grid(const TgqCoarse &c, long long tally)
 {
@@ -369,6 +447,13 @@ __device__ inline bool tgq_coarse_grid(const TgqCoarse &c, long long tally)
 	}
 	const long long mass_lo = (aq << 21) - (nz << 20);
 	return mass_lo - top >= (long long)tgq_acoef(n) << (TGQ_MASS_SHIFT - r);
+}
+
+// the class its producer gives a row: TGQ_CAND where a resolve has to decide
+__device__ inline int tgq_row_class(const TgqRowSums &s, int special)
+{
+	if (special) return TGQ_REF;
+	return tgq_candidate(s.tl) && !tgq_coarse_grid(s.co, s.tl) ? TGQ_CAND : TGQ_GRID;
 }
 
 // Resolves a candidate row of grid exponent E (a whole wave; h in LDS, this

@@ -1,0 +1,23 @@
+"""The decode step's fused norms and silu (four inputs a thread, digits and
+class from whole-wave sums) where quads, waves and blocks end: the decoder's
+logits against the fixed-length forward's, bit for bit."""
+import pytest
+
+from technograd_amd import hip
+from test_gpu_decode import check_decode
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def device():
+    print("gpu decode quads: tg_hip_init(0)", flush=True)
+    hip.init(0)
+
+
+# model width and MLP width: off quads, off 16-input groups, one wave and one
+# input more, the largest width, an MLP row of more than one pass of a block
+@pytest.mark.parametrize("D,FF,HD", [(50, 34, 16), (67, 99, 48), (256, 257, 32), (257, 1030, 128), (1023, 61, 256), (4096, 33, 16), (64, 4101, 64)])
+def test_widths_equal_fixed_length_forward(D, FF, HD):
+    print("case decode quads", D, FF, HD, flush=True)
+    check_decode(3, 5, 3, dict(L=2, D=D, NQ=2, NKV=1, HD=HD, FF=FF, V=96))
