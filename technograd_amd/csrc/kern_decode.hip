@@ -376,14 +376,11 @@ __global__ __launch_bounds__(256) void dec_hnorm_k(tgk_dec_hnorm_args a)
 			lane);
 }
 
-// Many lines at once (a prompt's token rows, or its head lines): a block of
-// NL_TPB threads holds R = NL_E / Kp whole lines, NL_EPT elements per thread
-// (all loaded before any is used), and the lines' R sequential sums of squares
-// run side by side, one thread each. Line L = t npr + j reads h + t hs + j D
-// (updated in place by modes 1 and 2, which need npr == 1), takes gain
-// g + j gs, writes out + L D and the digits of row L. The values are the
-// same as tgk_dec_norm's and tgk_dec_hnorm's: (h * inv) * g with
-// inv = 1 / sqrtf(sum / D + 1e-6), sum the ordered sum of the squares.
+// Many lines at once (a prompt's token rows, or its head lines). Line L = t
+// npr + j reads h + t hs + j D (updated in place by modes 1 and 2, which need
+// npr == 1), takes gain g + j gs, writes out + L D and the digits of row L.
+// The values are the same as tgk_dec_norm's and tgk_dec_hnorm's: (h * inv) *
+// g with inv = 1 / sqrtf(sum / D + 1e-6), sum the ordered sum of the squares.
 struct NormLines {
 	float *h;
 	long hs;
@@ -396,129 +393,198 @@ struct NormLines {
 	const float *g;
 	long gs;
 	float *out;
-	int D, Kp, npr;
-	long lines;
+	int D, npr;
+	int lines;
 	tgk_qdig q;
-	int kshift; // Kp = 1 << kshift
 };
-constexpr int NL_TPB = 256, NL_EPT = 16, NL_E = NL_TPB * NL_EPT;
 
-// LDS: R lines of Kp + 4 floats (16-byte aligned, consecutive lines 4 banks
-// apart), then per line its offsets, 1 / rms, exponent and flag
-size_t norm_lines_lds(int Kp) { return (size_t)(NL_E / Kp) * ((Kp + 4) * 4 + 8 + 4 * 4); }
-
-__global__ __launch_bounds__(NL_TPB) void norm_lines_k(NormLines a)
+// sums (or the max) over the LPL lanes of a line, in the last of them
+template <int LPL> __device__ inline int line_add(int v)
 {
+	v += tgq_dpp<0x111, 0xf>(v);
+	v += tgq_dpp<0x112, 0xf>(v);
+	v += tgq_dpp<0x114, 0xf>(v);
+	v += tgq_dpp<0x118, 0xf>(v);
+	if (LPL >= 32) v += tgq_dpp<0x142, 0xa>(v);
+	if (LPL >= 64) v += tgq_dpp<0x143, 0xc>(v);
+	return v;
+}
+template <int LPL> __device__ inline unsigned line_umax(unsigned v)
+{
+	v = max(v, (unsigned)tgq_dpp<0x111, 0xf>((int)v));
+	v = max(v, (unsigned)tgq_dpp<0x112, 0xf>((int)v));
+	v = max(v, (unsigned)tgq_dpp<0x114, 0xf>((int)v));
+	v = max(v, (unsigned)tgq_dpp<0x118, 0xf>((int)v));
+	if (LPL >= 32) v = max(v, (unsigned)tgq_dpp<0x142, 0xa>((int)v));
+	if (LPL >= 64) v = max(v, (unsigned)tgq_dpp<0x143, 0xc>((int)v));
+	return v;
+}
+// the same of lanes' sums of at most 64 |q|, which 64 lanes may take past 32 bits: by halves
+template <int LPL, int QPL> __device__ inline long long line_add_q(int v)
+{
+	if (LPL * QPL <= 64) return line_add<LPL>(v);
+	return (long long)line_add<LPL>(v >> 16) * 65536 + line_add<LPL>(v & 0xffff);
+}
+
+// A line is LPL lanes' with QPL quads a lane (quad s + LPL q is lane s's),
+// Kp = 4 LPL QPL; a wave holds 64 / LPL of them NL times over, in registers
+// from the load to the digits. Only the squares go through LDS, for the
+// ordered sums: one lane a line, the block's lines side by side in one wave,
+// another in each block (a block's first waves tend to share a SIMD, and the
+// sums' adds bound the kernel together with the memory). The digits go by
+// quads as in tgq_quad, a line's sums by data-parallel moves within its
+// lanes. FULL: D == Kp, no quad ends past the line.
+// 8192 rows of 1024 in 35 us (88 with one element a lane and access, every
+// value through LDS twice), 4.5 TB/s of 159 MB; 196,608 head lines of 128 in
+// 73 (118).
+template <int LPL, int QPL, int NL, bool FULL>
+__global__ __launch_bounds__(256) void norm_lines_k(NormLines a)
+{
+	constexpr int KP = 4 * LPL * QPL, G = 64 / LPL, LW = G * NL, R = 4 * LW, ZS = KP + 4;
 	extern __shared__ float4 sh4[];
-	const int Kp = a.Kp, D = a.D, ks = a.kshift, km = Kp - 1, R = NL_E >> ks, ZS = Kp + 4, tid = threadIdx.x;
-	float *z = (float *)sh4; // [R][ZS]: the squares, then the normalized values (0 from D on)
-	long *lh = (long *)(z + R * ZS); // line l's offset in h (t hs + j D)
-	int *lg = (int *)(lh + R), *lE = lg + R, *lsp = lE + R;
-	float *linv = (float *)(lsp + R);
-	const long L0 = (long)blockIdx.x * R;
-	if (tid < R) { // per line, once (lines past the end repeat the last)
-		const long L = L0 + tid < a.lines ? L0 + tid : a.lines - 1;
-		const long t = L / a.npr, j = L - t * a.npr;
-		lh[tid] = t * a.hs + j * D;
-		lg[tid] = (int)(j * a.gs);
-	}
-	__syncthreads();
-	// element u of this thread: e = tid + u NL_TPB, line e >> ks, column e & km
-	float v[NL_EPT];
-	for (int u = 0; u < NL_EPT; u++) {
-		const int e = tid + u * NL_TPB, l = e >> ks, i = e & km;
-		v[u] = a.h[lh[l] + (i < D ? i : D - 1)];
-	}
-	if (a.mode == 1) { // npr == 1: line l is token row L0 + l
-		float b[NL_EPT];
-		for (int u = 0; u < NL_EPT; u++) {
-			const int e = tid + u * NL_TPB, l = e >> ks, i = e & km;
-			const long L = L0 + l < a.lines ? L0 + l : a.lines - 1;
-			b[u] = a.add[L * a.adds + (i < D ? i : D - 1)];
-		}
-		for (int u = 0; u < NL_EPT; u++) v[u] = v[u] + b[u];
-	} else if (a.mode == 2) { // v + ((o_0 + o_1) + ... + o_{nh-1})
-		for (int u = 0; u < NL_EPT; u++) {
-			const int e = tid + u * NL_TPB, l = e >> ks, i = e & km;
-			const long L = L0 + l < a.lines ? L0 + l : a.lines - 1;
-			const float *o = a.o + L * D + (i < D ? i : D - 1);
-			float acc = o[0];
-			for (int k0 = 1; k0 < a.nh; k0 += 16) {
-				float b[16];
-				for (int k = 0; k < 16; k++) b[k] = o[(long)(k0 + k < a.nh ? k0 + k : 0) * a.ohead];
-				for (int k = 0; k < 16 && k0 + k < a.nh; k++) acc = acc + b[k];
+	float *z = (float *)sh4; // [R][ZS] squares; consecutive lines 4 banks apart
+	float *linv = z + R * ZS;
+	const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), sub = lane % LPL, grp = lane / LPL;
+	const int D = FULL ? KP : a.D, L0 = blockIdx.x * R, l0 = wave * LW + grp; // slot n: line L0 + l0 + n G
+	auto ld = [&](float *v, const float *p, int i) {
+		if (FULL) {
+			const f4u f = *(const f4u *)(p + i);
+			v[0] = f.x, v[1] = f.y, v[2] = f.z, v[3] = f.w;
+		} else
+			ld4(v, p, i, D);
+	};
+	auto st = [&](float *p, int i, const float *v) {
+		if (FULL) *(f4u *)(p + i) = f4u{ v[0], v[1], v[2], v[3] };
+		else st4(p, i, D, v);
+	};
+	float v[NL][QPL][4], g[NL][QPL][4];
+#pragma unroll
+	for (int n = 0; n < NL; n++) {
+		const int L = min(L0 + l0 + n * G, a.lines - 1), t = L / a.npr, j = L - t * a.npr; // (lines past the end read the last)
+#pragma unroll
+		for (int q = 0; q < QPL; q++) ld(v[n][q], a.h + (long)t * a.hs + (long)j * D, 4 * (sub + q * LPL));
+#pragma unroll
+		for (int q = 0; q < QPL; q++) ld(g[n][q], a.g + (long)j * a.gs, 4 * (sub + q * LPL));
+		if (a.mode == 1) { // npr == 1: line L is token row L
+			float b[QPL][4];
+#pragma unroll
+			for (int q = 0; q < QPL; q++) ld(b[q], a.add + (long)L * a.adds, 4 * (sub + q * LPL));
+#pragma unroll
+			for (int q = 0; q < QPL; q++)
+				for (int u = 0; u < 4; u++) v[n][q][u] = v[n][q][u] + b[q][u];
+		} else if (a.mode == 2) { // v + ((o_0 + o_1) + ... + o_{nh-1})
+#pragma unroll
+			for (int q = 0; q < QPL; q++) {
+				const float *o = a.o + (long)L * D;
+				float acc[4];
+				ld(acc, o, 4 * (sub + q * LPL));
+				for (int k = 1; k < a.nh; k++) {
+					float b[4];
+					ld(b, o + (long)k * a.ohead, 4 * (sub + q * LPL));
+					for (int u = 0; u < 4; u++) acc[u] = acc[u] + b[u];
+				}
+				for (int u = 0; u < 4; u++) v[n][q][u] = v[n][q][u] + acc[u];
 			}
-			v[u] = v[u] + acc;
 		}
 	}
-	for (int u = 0; u < NL_EPT; u++) {
-		const int e = tid + u * NL_TPB, l = e >> ks, i = e & km;
-		const bool in = L0 + l < a.lines && i < D;
-		if (in && a.mode) a.h[lh[l] + i] = v[u];
-		z[l * ZS + i] = in ? v[u] * v[u] : 0.0f;
+#pragma unroll
+	for (int n = 0; n < NL; n++) {
+		const int l = l0 + n * G;
+#pragma unroll
+		for (int q = 0; q < QPL; q++) {
+			const int i = 4 * (sub + q * LPL);
+			const float *x = v[n][q];
+			if (a.mode && L0 + l < a.lines) st(a.h + (long)(L0 + l) * a.hs, i, x);
+			*(float4 *)(z + l * ZS + i) = make_float4(x[0] * x[0], x[1] * x[1], x[2] * x[2], x[3] * x[3]);
+		}
 	}
 	__syncthreads();
-	if (tid < R && L0 + tid < a.lines) linv[tid] = 1.0f / sqrtf(tg_ordered_sum_pp<6>(z + tid * ZS, D) / (float)D + 1e-6f);
+	if (wave == (int)(blockIdx.x & 3) && lane < R) linv[lane] = 1.0f / sqrtf(tg_ordered_sum_pp<6>(z + lane * ZS, D) / (float)D + 1e-6f);
 	__syncthreads();
-	{
-		float gv[NL_EPT]; // the gains, all loaded before the first is used
-		for (int u = 0; u < NL_EPT; u++) {
-			const int e = tid + u * NL_TPB, l = e >> ks, i = e & km;
-			gv[u] = a.g[lg[l] + (i < D ? i : D - 1)];
+#pragma unroll
+	for (int n = 0; n < NL; n++) {
+		const int L = L0 + l0 + n * G;
+		const bool ok = L < a.lines;
+		const float inv = linv[l0 + n * G];
+		unsigned mb = 0;
+#pragma unroll
+		for (int q = 0; q < QPL; q++) {
+			const int i = 4 * (sub + q * LPL);
+			float *x = v[n][q];
+			for (int u = 0; u < 4; u++) x[u] = FULL || i + u < D ? x[u] * inv * g[n][q][u] : 0.0f;
+			if (ok) st(a.out + (long)L * D, i, x);
+			tgq_scan4(x, mb);
 		}
-		for (int u = 0; u < NL_EPT; u++) {
-			const int e = tid + u * NL_TPB, l = e >> ks, i = e & km;
-			const bool in = L0 + l < a.lines && i < D;
-			float nv = 0.0f;
-			if (in) {
-				nv = v[u] * linv[l] * gv[u];
-				a.out[(L0 + l) * D + i] = nv;
+		mb = (unsigned)__shfl((int)line_umax<LPL>(mb), lane | (LPL - 1));
+		float amax;
+		int nan;
+		tgq_scan_end(mb, amax, nan);
+		const int special = tgq_special(nan, amax), E = tgq_exponent(amax, special);
+		int8_t *blk = tgq_row_base(a.q.dig, L, KP);
+		int qs = 0, aq = 0, nx = 0; // a lane's at most 64 inputs: below 2^29
+#pragma unroll
+		for (int q = 0; q < QPL; q++) {
+			float *x = v[n][q];
+			unsigned u[4], w0, w1, w2;
+			for (int i = 0; i < 4; i++) {
+				if (special) x[i] = 0.0f; // zero digits, nothing to add up
+				const float sv = ldexpf(x[i], 23 - E), rq = rintf(sv);
+				const int qi = (int)rq;
+				qs += qi;
+				aq += abs(qi);
+				nx += rq != sv;
+				u[i] = (unsigned)(qi + 0x808080);
 			}
-			z[l * ZS + i] = nv;
+			tgq_pack4(u, w0, w1, w2);
+			const int k0 = 4 * (sub + q * LPL);
+			int8_t *p = blk + (k0 >> 5) * 3072 + ((k0 >> 4) & 1) * 512 + (k0 & 15);
+			if (ok) *(unsigned *)p = w0, *(unsigned *)(p + 1024) = w1, *(unsigned *)(p + 2048) = w2;
 		}
-	}
-	__syncthreads();
-	// per line: TPL = NL_TPB / R consecutive lanes (within one wave) take its max
-	// and flag, then its 16-input digit groups (Kp / 16 / TPL = 2 each) and
-	// the sum of their q, combined by shuffles
-	const int TPL = NL_TPB / R, l = tid / TPL, k = tid - l * TPL;
-	const float *zl = z + l * ZS;
-	float mx = 0.0f;
-	int bad = 0;
-	for (int m = k; m < Kp; m += TPL) {
-		const float x = zl[m];
-		bad |= !isfinite(x);
-		mx = fmaxf(mx, fabsf(x)); // a nan never wins fmaxf; such lines are flagged
-	}
-	for (int o = 1; o < TPL; o <<= 1) {
-		mx = fmaxf(mx, __shfl_xor(mx, o));
-		bad |= __shfl_xor(bad, o);
-	}
-	const int special = tgq_special(bad, mx), E = tgq_exponent(mx, special);
-	long long qs = 0, tl = 0;
-	if (L0 + l < a.lines) {
-		int8_t *blk = tgq_row_base(a.q.dig, (int)(L0 + l), Kp);
-		for (int gi = k; gi < Kp / 16; gi += TPL) {
-			float w16[16];
-			for (int q = 0; q < 16; q++) w16[q] = zl[gi * 16 + q];
-			qs += tgq_put16(blk, gi * 16, w16, E, special, tl);
+		TgqRowSums s{}; // (right in a line's last lane)
+		s.qs = line_add_q<LPL, QPL>(qs);
+		const long long ta = LPL * QPL <= 64 ? (long long)(unsigned)line_add<LPL>(aq) : line_add_q<LPL, QPL>(aq);
+		s.tl = ta + ((long long)line_add<LPL>(nx) << TGQ_TALLY_SHIFT);
+		const bool last = sub == LPL - 1;
+		if (__any(last && !special && tgq_candidate(s.tl))) { // the coarse test of candidate lines before any resolve
+			int n0 = 0, n1 = 0, nz = 0, a0 = 0, a1 = 0;
+#pragma unroll
+			for (int q = 0; q < QPL; q++)
+				for (int i = 0; i < 4; i++) {
+					const unsigned m = (unsigned)abs((int)rintf(ldexpf(v[n][q][i], 23 - E)));
+					const bool g0 = m >= (1u << 22), g1 = !g0 && m >= (1u << 21);
+					n0 += g0, n1 += g1, nz += v[n][q][i] != 0.0f;
+					a0 += g0 ? (int)m : 0, a1 += g1 ? (int)m : 0;
+				}
+			const int c01 = line_add<LPL>(n0 | n1 << 16), cz = line_add<LPL>(nz); // at most 4096 each
+			s.co.cnt = (unsigned long long)(c01 & 0xffff) + ((unsigned long long)(c01 >> 16) << 21) + ((unsigned long long)cz << 42);
+			s.co.s0 = LPL * QPL <= 64 ? (unsigned long long)(unsigned)line_add<LPL>(a0) : (unsigned long long)line_add_q<LPL, QPL>(a0);
+			s.co.s1 = LPL * QPL <= 64 ? (unsigned long long)(unsigned)line_add<LPL>(a1) : (unsigned long long)line_add_q<LPL, QPL>(a1);
 		}
+		if (last && ok) a.q.e[L] = E, a.q.special[L] = tgq_row_class(s, special), a.q.qsum[L] = s.qs;
 	}
-	for (int o = 1; o < TPL; o <<= 1) qs += __shfl_xor(qs, o), tl += __shfl_xor(tl, o);
-	int cls = special ? TGQ_REF : tgq_candidate(tl) ? TGQ_CAND : TGQ_GRID;
-	TgqCoarse co{}; // the coarse test of candidate lines before any resolve (shuffles within the line's lanes)
-	if (cls == TGQ_CAND)
-		for (int gi = k; gi < Kp / 16; gi += TPL) {
-			float w16[16];
-			for (int q = 0; q < 16; q++) w16[q] = zl[gi * 16 + q];
-			tgq_coarse16(co, w16, E);
-		}
-	for (int o = 1; o < TPL; o <<= 1)
-		co.cnt += __shfl_xor(co.cnt, o), co.s0 += __shfl_xor(co.s0, o), co.s1 += __shfl_xor(co.s1, o);
-	if (cls == TGQ_CAND && tgq_coarse_grid(co, tl)) cls = TGQ_GRID;
-	if (k == 0 && L0 + l < a.lines) {
-		const long L = L0 + l;
-		a.q.e[L] = E, a.q.special[L] = cls, a.q.qsum[L] = qs;
+}
+
+template <int LPL, int QPL, int NL> void norm_lines(hipStream_t s, const NormLines &n)
+{
+	constexpr int KP = 4 * LPL * QPL, R = 256 / LPL * NL;
+	const unsigned grid = (unsigned)(((long)n.lines + R - 1) / R);
+	const size_t lds = (size_t)R * (KP + 5) * sizeof(float);
+	if (n.D == KP) norm_lines_k<LPL, QPL, NL, true><<<grid, 256, lds, s>>>(n);
+	else norm_lines_k<LPL, QPL, NL, false><<<grid, 256, lds, s>>>(n);
+}
+
+// whether lines padded to Kp run there, and the launch
+// (4096: a block holds one line either way, and dec_norm_k is that kernel)
+bool norm_lines_for(hipStream_t s, int Kp, const NormLines &n)
+{
+	switch (Kp) {
+	case 64: norm_lines<16, 1, 4>(s, n); return true;
+	case 128: norm_lines<32, 1, 4>(s, n); return true;
+	case 256: norm_lines<64, 1, 4>(s, n); return true;
+	case 512: norm_lines<64, 2, 2>(s, n); return true;
+	case 1024: norm_lines<64, 4, 1>(s, n); return true;
+	case 2048: norm_lines<64, 8, 1>(s, n); return true;
+	default: return false;
 	}
 }
 
@@ -748,21 +814,15 @@ void tgk_dec_attn(hipStream_t s, const tgk_dec_attn_args *a, int seqs)
 
 // many lines (a prompt): norm_lines_k; few (a step): a block per row or a wave per head line
 constexpr long NL_MIN_LINES = 2048;
-inline bool nl_fits(int Kp) { return Kp >= 64 && Kp <= NL_E && (Kp & (Kp - 1)) == 0; } // a power of two: lines by shifts
-inline int ilog2(int x) { int k = 0; while ((1 << (k + 1)) <= x) k++; return k; }
-
 // threads of a block that takes a row of Kp values by fours
 inline unsigned quad_tpb(int Kp) { return Kp >= 4096 ? 1024u : (unsigned)(Kp + 255) / 256 * 64; }
 
 bool tgk_dec_norm(hipStream_t s, const tgk_dec_norm_args *a)
 {
 	if (a->rows <= 0) return true;
-	if (a->rows >= NL_MIN_LINES && nl_fits(a->Kp) && a->outs == a->D) {
-		NormLines n{ a->h, a->hs, a->mode, a->add, a->adds, a->o, a->ohead, a->nh, a->g, 0, a->out, a->D, a->Kp, 1, a->rows, a->q, ilog2(a->Kp) };
-		const long R = NL_E / a->Kp;
-		norm_lines_k<<<(unsigned)((a->rows + R - 1) / R), NL_TPB, norm_lines_lds(a->Kp), s>>>(n);
+	if (a->rows >= NL_MIN_LINES && a->outs == a->D &&
+	    norm_lines_for(s, a->Kp, NormLines{ a->h, a->hs, a->mode, a->add, a->adds, a->o, a->ohead, a->nh, a->g, 0, a->out, a->D, 1, a->rows, a->q }))
 		return false; // candidates left for tgk_qgemm_split
-	}
 	dec_norm_k<<<(unsigned)a->rows, quad_tpb(a->Kp), (size_t)a->Kp * 2 * sizeof(float), s>>>(*a);
 	return true;
 }
@@ -771,12 +831,9 @@ bool tgk_dec_hnorm(hipStream_t s, const tgk_dec_hnorm_args *a)
 {
 	const long lines = (long)a->rows * a->NH;
 	if (lines <= 0) return true;
-	if (lines >= NL_MIN_LINES && nl_fits(a->Kp)) {
-		NormLines n{ (float *)a->x, a->xs, 0, nullptr, 0, nullptr, 0, 0, a->g, a->HD, a->out, a->HD, a->Kp, a->NH, lines, a->q, ilog2(a->Kp) };
-		const long R = NL_E / a->Kp;
-		norm_lines_k<<<(unsigned)((lines + R - 1) / R), NL_TPB, norm_lines_lds(a->Kp), s>>>(n);
+	if (lines >= NL_MIN_LINES &&
+	    norm_lines_for(s, a->Kp, NormLines{ (float *)a->x, a->xs, 0, nullptr, 0, nullptr, 0, 0, a->g, a->HD, a->out, a->HD, a->NH, (int)lines, a->q }))
 		return false; // candidates left for tgk_qgemm_split
-	}
 	dec_hnorm_k<<<(unsigned)((lines + 3) / 4), TPB, (size_t)a->Kp * 4 * sizeof(float), s>>>(*a);
 	return true;
 }
