@@ -70,6 +70,33 @@ __global__ __launch_bounds__(256) void rope_cache4_k(tgk_dec_rope_args a, int ro
 	}
 }
 
+// Digits, exponent, class and sum of q of line L of K <= 256 inputs by one
+// wave, inputs 4 lane .. 4 lane + 3 in v (zeros from K on); z holds the line
+// in LDS for the resolve of a candidate that the coarse test leaves.
+__device__ inline void wave_digits(const float *v, const float *z, int K, int Kp, const tgk_qdig &q, int L, TgqHist *hist)
+{
+	const int lane = threadIdx.x & 63;
+	unsigned mb = 0;
+	tgq_scan4(v, mb);
+	mb = tgq_wave_umax(mb);
+	float amax;
+	int nan;
+	tgq_scan_end(mb, amax, nan);
+	const int special = tgq_special(nan, amax), E = tgq_exponent(amax, special);
+	int8_t *blk = tgq_row_base(q.dig, L, Kp);
+	TgqRowSums s{};
+	tgq_quad(blk, 4 * lane, 4 * lane < Kp, v, E, special, s);
+	const int cls = tgq_row_class(s, special);
+	if (lane == 0) q.e[L] = E, q.special[L] = cls, q.qsum[L] = s.qs;
+	if (cls != TGQ_CAND) return;
+	tgq_wave_sync();
+	const int nout = tgq_nout(Kp);
+	auto ld = [&](int g, float *x) {
+		for (int u = 0; u < 16; u++) x[u] = 16 * g + u < K ? z[16 * g + u] : 0.0f;
+	};
+	tgq_resolve_row(hist, ld, K, Kp, E, blk, &q.qsum[L], &q.e[L], &q.special[L], q.ok + (long)L * nout, q.ox + (long)L * nout, nout, lane);
+}
+
 // One decode step's attention: one block per (sequence, KV head) for the GRP
 // query heads sharing it, keys at positions 0 .. p. Per query head and key:
 // score = sum_d q[d] k[d] in order from 0.0f, times the scale, plus the mask's
@@ -84,6 +111,10 @@ __global__ __launch_bounds__(256) void rope_cache4_k(tgk_dec_rope_args a, int ro
 // a (key, head) thread per score, a (head, d) thread per output, carried
 // across chunks. LDS rows are HD + 4 floats apart: 16-byte reads of
 // consecutive rows by consecutive lanes hit distinct banks. HD % 16 == 0.
+// With Kp, a wave per query head then makes the digits of its outputs for the
+// output projections (line head rp + s): they are at hand, and a launch of
+// their own took a step 6.0 us a layer for 768 lines of 128; the attention
+// takes 2 more (26.4 to 28.4 us, 48 sequences at 232 positions on average).
 constexpr int ATT_TPB = 512, ATT_R = 4; // threads; float4 loads per thread and chunk
 
 int attn_chunk(int HD) // keys per chunk: ATT_R float4 loads per thread, at most 64
@@ -143,7 +174,7 @@ __global__ __launch_bounds__(ATT_TPB) void dec_attn_k(tgk_dec_attn_args a, int c
 	__syncthreads(); // the score chains are done with kv
 	stash();         // V's first chunk (fetched during the last K chunk) into kv,
 	if (ck < n) fetch(V, ck); // and its second in flight, both during the softmax
-	const int wave = tid >> 6, lane = tid & 63;
+	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
 	for (int g = wave; g < GRP; g += ATT_TPB >> 6) { // max: a wave per query head
 		const float *r = sc + g * nst;
 		float m = -INFINITY;
@@ -190,7 +221,14 @@ __global__ __launch_bounds__(ATT_TPB) void dec_attn_k(tgk_dec_attn_args a, int c
 		if (it >= GRP * HD) break;
 		const int g = it / HD, d = it - g * HD;
 		a.att[((long)s * a.NQ + j * GRP + g) * HD + d] = acc[u];
+		q[it] = acc[u];
 	}
+	if (!a.Kp) return;
+	__syncthreads(); // the heads' outputs are in q; kv is read, its room goes to the resolves (tgk_dec_attn_digits)
+	if (wave >= GRP) return;
+	const float4 o = 4 * lane < HD ? *(const float4 *)(q + wave * HD + 4 * lane) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+	const float v[4] = { o.x, o.y, o.z, o.w };
+	wave_digits(v, q + wave * HD, HD, a.Kp, a.q, (j * GRP + wave) * a.rp + s, (TgqHist *)kv + wave);
 }
 
 // four consecutive values of a line that starts at any float
@@ -354,26 +392,7 @@ __global__ __launch_bounds__(256) void dec_hnorm_k(tgk_dec_hnorm_args a)
 	for (int u = 0; u < 4; u++) nv[u] = i + u < HD ? v[u] * inv * g[u] : 0.0f;
 	st4(a.out + (long)L * HD, i, HD, nv);
 	if (i < Kp) *(float4 *)(z + i) = make_float4(nv[0], nv[1], nv[2], nv[3]);
-	unsigned mb = 0;
-	tgq_scan4(nv, mb);
-	mb = tgq_wave_umax(mb);
-	float amax;
-	int nan;
-	tgq_scan_end(mb, amax, nan);
-	const int special = tgq_special(nan, amax), E = tgq_exponent(amax, special);
-	int8_t *blk = tgq_row_base(a.q.dig, L, Kp);
-	TgqRowSums s{};
-	tgq_quad(blk, i, i < Kp, nv, E, special, s);
-	const int cls = tgq_row_class(s, special);
-	if (lane == 0) a.q.e[L] = E, a.q.special[L] = cls, a.q.qsum[L] = s.qs;
-	if (cls != TGQ_CAND) return;
-	tgq_wave_sync(); // the wave resolves its line (in z)
-	const int nout = tgq_nout(Kp);
-	auto ld = [&](int gi, float *x) {
-		for (int u = 0; u < 16; u++) x[u] = z[16 * gi + u];
-	};
-	tgq_resolve_row(&hist[w], ld, HD, Kp, E, blk, &a.q.qsum[L], &a.q.e[L], &a.q.special[L], a.q.ok + (long)L * nout, a.q.ox + (long)L * nout, nout,
-			lane);
+	wave_digits(nv, z, HD, Kp, a.q, L, &hist[w]);
 }
 
 // Many lines at once (a prompt's token rows, or its head lines). Line L = t
@@ -780,6 +799,11 @@ size_t tgk_dec_attn_lds(int GRP, int HD, int n)
 {
 	const long nst = (n + 3) & ~3;
 	return (size_t)((long)attn_chunk(HD) * (HD + 4) + (long)GRP * HD + GRP * nst + GRP) * sizeof(float);
+}
+
+bool tgk_dec_attn_digits(int GRP, int HD)
+{
+	return HD <= 256 && (size_t)GRP * sizeof(TgqHist) <= (size_t)attn_chunk(HD) * (HD + 4) * sizeof(float);
 }
 
 

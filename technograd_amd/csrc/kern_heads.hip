@@ -249,7 +249,7 @@ void tgk_heads(hipStream_t st, const tgk_heads_args *a, void *scratch)
 	tgk_qgemm_args g;
 	memset(&g, 0, sizeof g);
 	g.w = w, g.x = a->x, g.xr = a->xhead, g.xj = a->xrow, g.xk = 1, g.ni = a->rp, g.M = a->nh * a->rp;
-	tgk_qgemm_digits(st, &g, scratch);
+	if (!a->digits) tgk_qgemm_digits(st, &g, scratch);
 	const Heads d{ *a, tgk_qgemm_digit_area(scratch, g.M, w->Kp), (const int8_t *)w->w, w->scale, w->Kp, tgq_nout(w->Kp) };
 	// from 1024 rows 64 x 128 tiles fill a quarter of the chip and more; below, 16 x 16 tiles with the heads side by side
 	if (a->rows >= 1024) {

@@ -212,6 +212,8 @@ bool forward(tg_hip_dec *d, int S, int T0, int p0)
 	const int rows = S * T0, NH = d->NQ + d->NKV, GRP = d->NQ / d->NKV;
 	const long ctot = (long)(d->NQ + 2 * d->NKV) * d->HD, qk = (long)NH * d->HD, D = d->D;
 	hipStream_t st = d->st;
+	const int rp = (rows + 31) / 32 * 32;
+	const bool head_digits = heads_fused(d) && T0 == 1 && tgk_dec_attn_digits(GRP, d->HD); // by the attention, for the output projections
 	tgk_take(st, d->h, (long)T0 * D, tgk_opd{ d->E, 0 }, tgk_opd{ d->ids, T0 }, T0, d->V, d->D, S);
 	for (int l = 0; l < d->L; l++) {
 		const long kv_layer = (long)l * d->S * d->kv_seq; // the cache is layer-major: [layer][sequence][KV head][position][HD]
@@ -233,6 +235,8 @@ bool forward(tg_hip_dec *d, int S, int T0, int p0)
 			tgk_dec_attn_args a;
 			a.qr = d->qr, a.K = d->K, a.V = d->Vc, a.att = d->att, a.kv_seq = d->kv_seq, a.kv_layer = kv_layer;
 			a.NQ = d->NQ, a.NKV = d->NKV, a.HD = d->HD, a.P = d->P, a.p = p0, a.scale = d->scale;
+			a.Kp = head_digits ? d->ws[(size_t)d->wo[(size_t)l]].Kp : 0, a.rp = rp;
+			if (head_digits) a.q = tgk_qgemm_digit_area(d->scratch, d->NQ * rp, a.Kp);
 			tgk_dec_attn(st, &a, S);
 		} else { // a prompt from position 0: the graph's products, scale, mask and softmax (causal), the heads that
 			// the score buffer holds in one launch (a head alone leaves the chip half empty)
@@ -264,7 +268,7 @@ bool forward(tg_hip_dec *d, int S, int T0, int p0)
 		// TGK_REFLOOP_K take the reference's loop, as every short product does: a product per head, summed by the norm
 		if (heads_fused(d)) {
 			tgk_heads_args ha;
-			ha.x = d->att, ha.xrow = (long)d->NQ * d->HD, ha.xhead = d->HD, ha.rows = rows, ha.rp = (rows + 31) / 32 * 32;
+			ha.x = d->att, ha.xrow = (long)d->NQ * d->HD, ha.xhead = d->HD, ha.rows = rows, ha.rp = rp, ha.digits = head_digits;
 			ha.nh = d->NQ, ha.HD = d->HD, ha.D = d->D, ha.Dp = (d->D + 255) / 256 * 256;
 			ha.w = &d->ws[(size_t)d->wo[(size_t)l]], ha.o = d->dbuf, ha.orow = D;
 			tgk_heads(st, &ha, d->scratch);

@@ -166,7 +166,11 @@ typedef struct {
 	long kv_seq, kv_layer;
 	int NQ, NKV, HD, P, p;    /* keys at positions 0 .. p */
 	float scale;
+	int Kp, rp;               /* Kp: also the digits of head h of sequence s, as line h rp + s padded to Kp (0: none) */
+	tgk_qdig q;
 } tgk_dec_attn_args;
+/* whether the attention's block has room to make its outputs' digits */
+bool tgk_dec_attn_digits(int GRP, int HD);
 /* LDS bytes of one step's attention block for n keys (at most 65536 to launch) */
 size_t tgk_dec_attn_lds(int GRP, int HD, int n);
 void tgk_dec_attn(hipStream_t s, const tgk_dec_attn_args *a, int seqs);
@@ -233,6 +237,7 @@ typedef struct {
 	const tgk_qweight *w;
 	float *o;
 	long orow;
+	int digits; /* the scratch holds the lines' digits already (line head rp + row; those of padding rows may be anything) */
 } tgk_heads_args;
 void tgk_heads(hipStream_t s, const tgk_heads_args *a, void *scratch);
 /* causal softmax over a prompt chunk's scores sc [lines][T0] (line L is

@@ -29,3 +29,11 @@ def test_widths_equal_fixed_length_forward(D, FF, HD):
 def test_many_lines_equal_fixed_length_forward(seqs, T0, D, HD):
     print("case many lines", seqs, T0, D, HD, flush=True)
     check_decode(seqs, T0, 2, dict(L=2, D=D, NQ=2, NKV=1, HD=HD, FF=64, V=96))
+
+
+# the attention's digits for the output projections: sequences off the 32-row blocks, 1 to 8 query heads a KV head (8 of
+# 48 do not fit the block's room and take the digit kernel), the largest and smallest heads, a one-token prompt
+@pytest.mark.parametrize("seqs,T0,NQ,NKV,HD", [(33, 3, 4, 4, 48), (2, 1, 8, 1, 48), (37, 2, 8, 1, 64), (31, 4, 8, 2, 256), (3, 70, 2, 1, 144)])
+def test_attention_digits_equal_fixed_length_forward(seqs, T0, NQ, NKV, HD):
+    print("case attention digits", seqs, T0, NQ, NKV, HD, flush=True)
+    check_decode(seqs, T0, 3, dict(L=2, D=96, NQ=NQ, NKV=NKV, HD=HD, FF=64, V=96))
