@@ -2636,7 +2636,10 @@ int batch_host(tg_hip_prog *p, const void *rows, long nrows, void *out, int *ste
 		const long i = arrived, r0 = i * C, cnt = nrows - r0 < C ? nrows - r0 : C;
 		const int k = (int)(i % NSL);
 		const hipError_t e = wait ? hipEventSynchronize(h.down[k]) : hipEventQuery(h.down[k]);
-		if (e == hipErrorNotReady) return true;
+		if (e == hipErrorNotReady) {
+			(void)hipGetLastError(); // an answer, not an error: the next pass's launch check must not find it
+			return true;
+		}
 		if (!hipok(e, "outputs to host")) return false;
 		if (!dout) p->copies.submit((char *)out + (size_t)r0 * nout * 4, h.h_out[k], (size_t)cnt * nout * 4, CopyPool::OUT_PIECE, left.out[k]);
 		if (steps && p->m->nthink && !dsteps) memcpy(steps + (size_t)r0 * nt, h.h_steps[k], (size_t)cnt * nt * 4);

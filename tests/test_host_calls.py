@@ -1,0 +1,60 @@
+"""The library's host code around the device (chunks, slots, error paths,
+allocations) on a host without one: tests/cpp/fake_device.cpp answers the HIP
+calls in host memory and checks every copy against its allocations. Kernels do
+nothing there, so these tests look at what is asked of the device, not at
+values. Each runs in a process of its own, where the runtime is preloaded."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+ROCM = "/opt/rocm/include"
+
+pytestmark = pytest.mark.skipif(not shutil.which("g++") or not os.path.exists(ROCM + "/hip/hip_runtime_api.h"), reason="no g++ or HIP headers")
+
+HEAD = """
+import ctypes, gc, os, sys
+import numpy as np
+sys.path.insert(0, %r)
+from technograd_amd import hip, synth
+fake = ctypes.CDLL(os.environ["FAKE_DEVICE"])
+for f in ("fake_pending", "fake_out_of_range", "fake_launches", "fake_used", "fake_largest"):
+    getattr(fake, f).restype = ctypes.c_long
+for f in ("fake_fail_launch", "fake_limit"):
+    getattr(fake, f).argtypes = [ctypes.c_long]
+hip.init(0)
+def linear(k, c):
+    return synth.linear_tgir("m", synth.rand(1, 0.05, c * k).reshape(c, k), 8)
+def pinned(a):
+    hb = hip.HostBuffer(max(a.nbytes, 1))
+    v = hb.array(a.dtype, a.shape)
+    v[:] = a
+    return hb, v
+""" % ROOT
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "fake_device.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I" + ROCM, "-o", so, os.path.join(ROOT, "tests", "cpp", "fake_device.cpp")], check=True)
+
+    def go(code):
+        env = dict(os.environ, FAKE_DEVICE=so, LD_PRELOAD=":".join(filter(None, (so, os.environ.get("LD_PRELOAD")))))
+        r = subprocess.run([sys.executable, "-c", HEAD + code], env=env, capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0, (r.stdout[-2000:], r.stderr[-3000:])
+    return go
+
+
+def test_a_chunk_not_down_yet_is_no_error(run):
+    """Asking for a chunk that is still on its way leaves "not ready" as the
+    runtime's last error, which the launch check of the next pass must not
+    report."""
+    run("""
+prog = hip.Program(linear(64, 40), max_rows=7)
+for n in (8, 29, 200):
+    y, _ = prog.batch(np.ones((n, 64), np.float32))
+    assert fake.fake_out_of_range() == 0 and fake.fake_pending() == 0
+""")
