@@ -1993,6 +1993,10 @@ void run_fixed_steps(tg_hip_prog *p, int lo, int hi, int t, int rows, int *d_ste
 
 int run_pass(tg_hip_prog *p, const float *d_in, int rows, float *d_out, int *d_steps)
 {
+	if (rows > p->max_rows) { // the arena and the scratch hold no more
+		seterr("a pass of %d rows exceeds the program's %d-row capacity", rows, p->max_rows);
+		return -1;
+	}
 	if (p->fx_steps) {
 		if (rows <= 0) return 0;
 		tgk_fx_in(p->st, (int *)p->d_arena + (long)p->rp_in_slot * p->max_rows, p->max_rows, (const int *)d_in, (int)p->m->per, rows);
@@ -2612,9 +2616,9 @@ int batch_host(tg_hip_prog *p, const void *rows, long nrows, void *out, int *ste
 	const long per = p->m->per, nout = p->m->nout, nt = p->m->nthink ? p->m->nthink : 1;
 	const bool din = in_pinned(rows, (size_t)nrows * per * 4), dout = in_pinned(out, (size_t)nrows * nout * 4);
 	const bool dsteps = steps && in_pinned(steps, (size_t)nrows * nt * 4);
-	// equal chunks of at most h.chunk rows, half that for what nothing stages, so that what nothing overlaps (the first
-	// one's way in, the last one's way out) is short
-	const long cmax = din && dout ? std::max(64L, (h.chunk + 1) / 2) : h.chunk;
+	// equal chunks of at most h.chunk rows (what a slot and a pass hold), half that, from 64 rows on, for what nothing
+	// stages, so that what nothing overlaps (the first one's way in, the last one's way out) is short
+	const long cmax = din && dout ? std::min(h.chunk, std::max(64L, (h.chunk + 1) / 2)) : h.chunk;
 	const long nch0 = (nrows + cmax - 1) / cmax, C = nch0 > 1 ? (nrows + nch0 - 1) / nch0 : cmax, nch = (nrows + C - 1) / C;
 	const hipStream_t up = nch > 1 ? h.h2d : p->st, down = nch > 1 ? h.d2h : p->st;
 	float ms_total = 0;

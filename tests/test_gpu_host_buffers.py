@@ -83,3 +83,22 @@ def test_pageable_rows_in_one_chunk_and_many():
         got, steps = prog.batch(x[:rows])
         assert np.array_equal(got.view(np.uint32), want[:rows].view(np.uint32)) and not steps.any()
     prog.close()
+
+
+@pytest.mark.parametrize("max_rows", [1, 7, 33])
+def test_pinned_rows_in_passes_of_a_small_program(max_rows):
+    """Pinned rows and outputs through a program of few rows a pass: passes of
+    at most that many, the bits of the same rows one pass at a time."""
+    print("case small pinned", max_rows, flush=True)
+    text = synth.linear_tgir("small", synth.rand(1, 0.05, 40 * 64).reshape(40, 64), 8)
+    n = 2 * max_rows + 65
+    x = synth.rand(4, 1.0, n * 64).reshape(n, 64).astype(np.float32)
+    prog = hip.Program(text, max_rows=max_rows)
+    want = np.concatenate([prog.batch(x[a:a + max_rows])[0] for a in range(0, n, max_rows)])
+    bx, px = pinned_like(x)
+    by, py = pinned_like(np.zeros((n, 40), np.float32))
+    got, _ = prog.batch(px, py)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    for b in (bx, by):
+        b.free()
+    prog.close()
