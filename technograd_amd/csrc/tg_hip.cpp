@@ -2622,19 +2622,24 @@ int batch_host(tg_hip_prog *p, const void *rows, long nrows, void *out, int *ste
 	const long nch0 = (nrows + cmax - 1) / cmax, C = nch0 > 1 ? (nrows + nch0 - 1) / nch0 : cmax, nch = (nrows + C - 1) / C;
 	const hipStream_t up = nch > 1 ? h.h2d : p->st, down = nch > 1 ? h.d2h : p->st;
 	float ms_total = 0;
-	struct Left { // pieces of each slot's copies; none outlives the call, whatever it returns
-		CopyPool &pool;
+	// Pieces of each slot's copies; neither they nor anything queued on the device outlives the call, whatever it
+	// returns: an error part way leaves transfers that write the caller's buffers or the slots of the next call.
+	struct Left {
+		tg_hip_prog *p;
+		bool down = false; // every chunk is
 		std::atomic<int> in{ 0 }, out[NSL];
-		Left(CopyPool &c) : pool(c)
+		Left(tg_hip_prog *p_) : p(p_)
 		{
 			for (auto &x : out) x = 0;
 		}
 		~Left()
 		{
-			pool.wait(in);
-			for (auto &x : out) pool.wait(x);
+			if (!down)
+				for (hipStream_t s : { p->hp.h2d, p->st, p->hp.d2h }) (void)hipStreamSynchronize(s);
+			p->copies.wait(in);
+			for (auto &x : out) p->copies.wait(x);
 		}
-	} left(p->copies);
+	} left(p);
 	long arrived = 0; // chunks before it are down, their copies to the caller begun
 	auto arrive = [&](bool wait) -> bool { // the next chunk's outputs, if they are down (or once they are)
 		const long i = arrived, r0 = i * C, cnt = nrows - r0 < C ? nrows - r0 : C;
@@ -2687,6 +2692,7 @@ int batch_host(tg_hip_prog *p, const void *rows, long nrows, void *out, int *ste
 	}
 	while (arrived < nch)
 		if (!arrive(true)) return -1;
+	left.down = true;
 	for (auto &x : left.out) p->copies.wait(x);
 	collect_timing(p);
 	if (steps && !p->m->nthink) memset(steps, 0, (size_t)nrows * sizeof *steps); /* no think loop: one zero slot per row */

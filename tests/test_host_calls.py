@@ -71,3 +71,28 @@ for n in (1, 2, 32, 63, 64, 65, 129, 500):
     assert fake.fake_pending() == 0, n
     bx.free(), by.free()
 """ % max_rows)
+
+
+@pytest.mark.parametrize("pin", [False, True])
+def test_nothing_is_in_flight_after_an_error(run, pin):
+    """A pass that fails part way through a batch: when the call has returned
+    its error, no transfer is left that could write the caller's memory or the
+    slots of the next call, and the next call works."""
+    run("""
+prog = hip.Program(linear(64, 40), max_rows=70)
+(bx, x), (by, y) = pinned(np.ones((500, 64), np.float32)), pinned(np.zeros((500, 40), np.float32))
+if not %r:
+    x, y = np.array(x), np.array(y)
+first = fake.fake_launches()
+prog.batch(x, y)
+for n in range(1, fake.fake_launches() - first + 1):
+    fake.fake_fail_launch(n)
+    try:
+        prog.batch(x, y)
+        raise SystemExit("launch %%d of the batch failed without an error" %% n)
+    except RuntimeError:
+        pass
+    assert fake.fake_pending() == 0, n
+    prog.batch(x, y)
+    assert fake.fake_pending() == 0 and fake.fake_out_of_range() == 0
+""" % pin)
