@@ -43,6 +43,7 @@
 #include <cstring>
 #include <deque>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <system_error>
@@ -175,12 +176,13 @@ struct Step {
 	int qv = -1, seg = -1;
 };
 
-// Host threads of one program's host-buffer batches, copying pieces between
-// the caller's pageable buffers and the pinned slots: made at the first copy
-// that is worth sharing, kept between calls (making eight takes 80 us, as
-// long as the copy of a chunk), joined when the program is freed. A worker
-// that finds nothing to do looks again for a while before it sleeps, so that
-// within a batch the next piece does not wait for a wake-up.
+// Host threads of the host-buffer batches, copying pieces between the
+// callers' pageable buffers and the pinned slots: made at the first copy that
+// is worth sharing, kept between calls (making eight takes 80 us, as long as
+// the copy of a chunk), shared by all programs (copy_pool) and joined when the
+// last program that has run such a batch is freed. A worker that finds
+// nothing to do looks again for a while before it sleeps, so that within a
+// batch the next piece does not wait for a wake-up.
 class CopyPool {
 	struct Piece {
 		char *dst;
@@ -211,6 +213,7 @@ class CopyPool {
 	}
 	void start()
 	{
+		std::lock_guard<std::mutex> lk(mu);
 		if (started) return;
 		started = true;
 		const unsigned hc = std::thread::hardware_concurrency();
@@ -281,6 +284,17 @@ public:
 	}
 };
 
+// the process's one pool, while a program holds it
+std::shared_ptr<CopyPool> copy_pool()
+{
+	static std::mutex mu;
+	static std::weak_ptr<CopyPool> pool;
+	std::lock_guard<std::mutex> lk(mu);
+	std::shared_ptr<CopyPool> p = pool.lock();
+	if (!p) pool = p = std::make_shared<CopyPool>();
+	return p;
+}
+
 } // namespace
 
 struct tg_hip_prog {
@@ -327,7 +341,7 @@ struct tg_hip_prog {
 	std::string rp_why;            // why the program runs in the interpreter
 	// host-buffer batches: a pipeline of slots (pinned staging, device buffers, copy streams, events)
 	static constexpr int NSL = 4;
-	CopyPool copies;
+	std::shared_ptr<CopyPool> copies; // from the first host-buffer batch on
 	struct HostPipe {
 		long chunk = 0;                                            // rows per chunk
 		void *h_in[NSL] = {}, *h_out[NSL] = {};                    // pinned staging
@@ -2568,6 +2582,7 @@ bool host_pipe_init(tg_hip_prog *p)
 {
 	auto &h = p->hp;
 	if (h.chunk) return true;
+	p->copies = copy_pool();
 	const long per = p->m->per, nout = p->m->nout, nt = p->m->nthink ? p->m->nthink : 1;
 	// up to 8 MiB of rows per chunk: smaller ones travel as well (4 MiB: 51 GB/s, 16 MiB: 56) but compute less well
 	// (2048 rows of a 512-2048-2048-512 MLP 180 us, 4096 of them 200)
@@ -2636,8 +2651,8 @@ int batch_host(tg_hip_prog *p, const void *rows, long nrows, void *out, int *ste
 		{
 			if (!down)
 				for (hipStream_t s : { p->hp.h2d, p->st, p->hp.d2h }) (void)hipStreamSynchronize(s);
-			p->copies.wait(in);
-			for (auto &x : out) p->copies.wait(x);
+			p->copies->wait(in);
+			for (auto &x : out) p->copies->wait(x);
 		}
 	} left(p);
 	long arrived = 0; // chunks before it are down, their copies to the caller begun
@@ -2650,7 +2665,7 @@ int batch_host(tg_hip_prog *p, const void *rows, long nrows, void *out, int *ste
 			return true;
 		}
 		if (!hipok(e, "outputs to host")) return false;
-		if (!dout) p->copies.submit((char *)out + (size_t)r0 * nout * 4, h.h_out[k], (size_t)cnt * nout * 4, CopyPool::OUT_PIECE, left.out[k]);
+		if (!dout) p->copies->submit((char *)out + (size_t)r0 * nout * 4, h.h_out[k], (size_t)cnt * nout * 4, CopyPool::OUT_PIECE, left.out[k]);
 		if (steps && p->m->nthink && !dsteps) memcpy(steps + (size_t)r0 * nt, h.h_steps[k], (size_t)cnt * nt * 4);
 		float ms = 0;
 		(void)hipEventElapsedTime(&ms, h.t0[k], h.t1[k]);
@@ -2663,12 +2678,12 @@ int batch_host(tg_hip_prog *p, const void *rows, long nrows, void *out, int *ste
 		const long r0 = i * C, cnt = nrows - r0 < C ? nrows - r0 : C;
 		if (i >= NSL) { // the slot's previous chunk is out: its buffers are free
 			if (arrived <= i - NSL && !arrive(true)) return -1;
-			p->copies.wait(left.out[k]);
+			p->copies->wait(left.out[k]);
 		}
 		const void *src = (const char *)rows + (size_t)r0 * per * 4;
 		if (!din) {
-			p->copies.submit(h.h_in[k], src, (size_t)cnt * per * 4, CopyPool::IN_PIECE, left.in);
-			p->copies.wait(left.in);
+			p->copies->submit(h.h_in[k], src, (size_t)cnt * per * 4, CopyPool::IN_PIECE, left.in);
+			p->copies->wait(left.in);
 			src = h.h_in[k];
 		}
 		if (!hipok(hipMemcpyAsync(h.d_in[k], src, (size_t)cnt * per * 4, hipMemcpyHostToDevice, up), "rows to device")) return -1;
@@ -2693,7 +2708,7 @@ int batch_host(tg_hip_prog *p, const void *rows, long nrows, void *out, int *ste
 	while (arrived < nch)
 		if (!arrive(true)) return -1;
 	left.down = true;
-	for (auto &x : left.out) p->copies.wait(x);
+	for (auto &x : left.out) p->copies->wait(x);
 	collect_timing(p);
 	if (steps && !p->m->nthink) memset(steps, 0, (size_t)nrows * sizeof *steps); /* no think loop: one zero slot per row */
 	p->stats.rows = (int)nrows;

@@ -96,3 +96,35 @@ for n in range(1, fake.fake_launches() - first + 1):
     prog.batch(x, y)
     assert fake.fake_pending() == 0 and fake.fake_out_of_range() == 0
 """ % pin)
+
+
+def test_programs_share_their_copy_threads(run):
+    """Any number of programs that copy pageable rows hold one set of host
+    threads, also while several run, and none once they are freed."""
+    run("""
+import threading
+def threads():
+    return len(os.listdir("/proc/self/task"))
+base = threads()
+x = np.ones((9000, 64), np.float32)  # 2.3 MB: copies worth sharing
+progs = [hip.Program(linear(64, 64), max_rows=9000) for _ in range(12)]
+for p in progs:
+    p.batch(x)
+assert threads() <= base + 11, (base, threads())
+calls = [threading.Thread(target=lambda p=p: [p.batch(x) for _ in range(20)]) for p in progs]
+for t in calls:
+    t.start()
+for t in calls:
+    t.join()
+assert threads() <= base + 11, (base, threads())
+for p in progs[:-1]:
+    p.close()
+y, _ = progs[-1].batch(x)  # the last one still has them
+progs[-1].close()
+assert threads() == base, (base, threads())
+progs = [hip.Program(linear(64, 64), max_rows=9000) for _ in range(2)]
+for p in progs:
+    p.batch(x)
+    p.close()
+assert threads() == base, (base, threads())
+""")
