@@ -2065,6 +2065,10 @@ int tgk_qweight_pack(tgk_qweight *w, const uint8_t *codes, const float *scale, i
 		    hipMemcpyAsync(w->scale, hs, (size_t)w->Cp * sizeof(float), hipMemcpyHostToDevice, st) != hipSuccess ||
 		    hipMemcpyAsync(w->orig, codes, ob, hipMemcpyHostToDevice, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess))
 		rc = -1;
+	if (rc) { // the caller reports it
+		tgk_qweight_free(w);
+		(void)hipGetLastError();
+	}
 	free(h);
 	free(hs);
 	free(hg);

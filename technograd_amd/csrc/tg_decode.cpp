@@ -71,6 +71,7 @@ bool hip_ok(hipError_t e, const char *what)
 	char buf[256];
 	snprintf(buf, sizeof buf, "%s: %s", what, hipGetErrorString(e));
 	tgh_set_error(buf);
+	(void)hipGetLastError(); // reported here: the next launch check must not report it again
 	return false;
 }
 

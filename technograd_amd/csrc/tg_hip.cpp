@@ -66,6 +66,7 @@ bool hipok(hipError_t e, const char *what)
 {
 	if (e == hipSuccess) return true;
 	seterr("%s: %s", what, hipGetErrorString(e));
+	(void)hipGetLastError(); // reported here: the next launch check must not report it again
 	return false;
 }
 

@@ -128,3 +128,27 @@ for p in progs:
     p.close()
 assert threads() == base, (base, threads())
 """)
+
+
+def test_an_error_is_reported_once(run):
+    """A program or decoder that does not fit the device's memory is refused,
+    leaves none of it taken, and the calls after it are not refused for it."""
+    run("""
+prog = hip.Program(linear(64, 40), max_rows=7)
+x = np.ones((20, 64), np.float32)
+prog.batch(x)
+qwen = hip.Program(synth.qwen3_tgir("q", T=8, rope_len=70, L=1, D=64, NQ=4, NKV=2, HD=64, FF=96, V=320), max_rows=1)
+big, used = linear(512, 512), fake.fake_used()
+for make in (lambda: hip.Program(big, max_rows=4096), lambda: hip.Decoder(qwen, 4, 64, 70)):
+    for left in (4096, 1 << 15, 1 << 17, 300000, 1 << 19, 1 << 20):
+        fake.fake_limit(used + left)
+        try:
+            make()
+            raise SystemExit("made in %d bytes" % left)
+        except RuntimeError:
+            pass
+        gc.collect()
+        assert fake.fake_used() == used, (left, fake.fake_used() - used)
+        prog.batch(x)
+    fake.fake_limit(1 << 40)
+""")
