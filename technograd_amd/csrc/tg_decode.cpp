@@ -372,8 +372,6 @@ bool build(tg_hip_dec *d)
 	if (d->wrot < 0 || d->wlm < 0) return err("decoder: cannot place Rot or the LM head");
 	// cache and buffers
 	const long rows = (long)d->S * d->TP;
-	const long sc1 = (long)d->S * d->TP * d->TP;
-	d->sc_floats = std::max(sc1, std::min(sc1 * d->NQ, SC_MAX));
 	d->kv_seq = (long)d->NKV * d->P * HD; // one sequence's K (or V) of one layer; a layer holds S of them
 	if (!alloc(d, &d->K, (size_t)(d->L * d->S * d->kv_seq)) || !alloc(d, &d->Vc, (size_t)(d->L * d->S * d->kv_seq)) || !alloc(d, &d->ids, (size_t)rows) ||
 	    !alloc(d, &d->h, (size_t)(rows * d->D)) ||
@@ -382,7 +380,6 @@ bool build(tg_hip_dec *d)
 	    !alloc(d, &d->att, (size_t)((rows + 31) / 32 * 32 * d->NQ * HD)) ||
 	    !alloc(d, &d->wout, heads_fused(d) ? 0 : (size_t)(rows * d->NQ * d->D)) ||
 	    !alloc(d, &d->gu, (size_t)(rows * 2 * d->FF)) || !alloc(d, &d->act, (size_t)(rows * d->FF)) || !alloc(d, &d->dbuf, (size_t)(rows * d->D)) ||
-	    !alloc(d, &d->sc, (size_t)d->sc_floats) ||
 	    !alloc(d, &d->lastn, (size_t)((long)d->S * d->D)) || !alloc(d, &d->logits, (size_t)((long)d->S * d->V)) ||
 	    !alloc(d, &d->am_v, (size_t)d->S * TGK_AM_PARTS) || !alloc(d, &d->am_i, (size_t)d->S * TGK_AM_PARTS))
 		return false;
@@ -392,7 +389,15 @@ bool build(tg_hip_dec *d)
 	need(rows, d->wqkv[0]), need(rows * NH, d->wrot), need(heads_fused(d) ? rp * d->NQ : rows, d->wo[0]), need(rows, d->wgu[0]), need(rows, d->wd[0]), need(d->S, d->wlm);
 	d->scratch_bytes = sb;
 	if (!hip_ok(hipMemsetAsync(d->att, 0, (size_t)(rp * d->NQ * HD) * sizeof(float), d->st), "decoder memory")) return false; // (its padding rows are read)
-	return hip_ok(hipMalloc(&d->scratch, sb), "decoder scratch") && hip_ok(hipStreamSynchronize(d->st), "decoder upload");
+	if (!hip_ok(hipMalloc(&d->scratch, sb), "decoder scratch")) return false;
+	// a prompt's scores, last: as many heads' as SC_MAX and the memory that is left hold, one head's at least
+	const long sc1 = (long)d->S * d->TP * d->TP;
+	for (long n = std::max(sc1, std::min(sc1 * d->NQ, SC_MAX));; n = std::max(sc1, n / 2)) {
+		d->sc_floats = n;
+		if (alloc(d, &d->sc, (size_t)n)) break;
+		if (n == sc1) return false;
+	}
+	return hip_ok(hipStreamSynchronize(d->st), "decoder upload");
 }
 
 } // namespace

@@ -152,3 +152,37 @@ for make in (lambda: hip.Program(big, max_rows=4096), lambda: hip.Decoder(qwen, 
         prog.batch(x)
     fake.fake_limit(1 << 40)
 """)
+
+
+def test_decoder_needs_no_more_than_one_heads_scores(run):
+    """Scores of all heads at once are taken where they fit: with less device
+    memory left the decoder keeps fewer heads' and runs the rest of them in
+    further launches, down to one head's."""
+    run("""
+S, T0, NQ = 2, 256, 8
+prog = hip.Program(synth.qwen3_tgir("q", T=8, rope_len=T0 + 2, L=1, D=64, NQ=NQ, NKV=2, HD=64, FF=96, V=320), max_rows=1)
+base, head = fake.fake_used(), 4 * S * T0 * T0
+prompt, tokens = hip.DeviceBuffer(4 * S * T0), hip.DeviceBuffer(8 * S)
+def make(left):
+    fake.fake_limit(fake.fake_used() + left)
+    dec = hip.Decoder(prog, S, T0, T0 + 2)
+    used, n = fake.fake_used(), fake.fake_launches()
+    dec.generate_device(prompt.ptr, S, T0, 2, tokens.ptr, None)  # (the failed allocations are not its launch error)
+    prog.sync()
+    assert fake.fake_out_of_range() == 0
+    n = fake.fake_launches() - n
+    dec.close()
+    return used - base, n
+base = fake.fake_used()
+full, launches = make(1 << 40)
+least = full - (NQ - 1) * head
+for heads in (1, 2, 3, 4, 7):
+    used, n = make(least + (heads - 1) * head)
+    assert used <= least + (heads - 1) * head and n > launches, (heads, used, n, launches)
+try:
+    make(least - 1)
+    raise SystemExit("a decoder in less memory than it needs")
+except RuntimeError as e:
+    assert "out of memory" in str(e)
+assert make(1 << 40) == (full, launches)
+""")
