@@ -79,51 +79,59 @@ __device__ inline float line_value(const Heads &d, int h, int row, int c, int E,
 
 // A step's rows: a block per 16 rows x 16 channels, a wave per head (in
 // turns), whose digits and weights all load at once into
-// v_mfma_i32_16x16x64_i8's operands; the heads' values meet in LDS and 256
-// threads add them in order. A head's product is a load's latency and six
-// matrix instructions; what bounds the kernel is the bytes a compute unit
-// takes in (128 KB a block at 16 heads of 128).
+// v_mfma_i32_16x16x64_i8's operands; the heads' values meet in LDS, HG heads'
+// at a time, and 256 threads add them in order. A head's product is a load's
+// latency and six matrix instructions; what bounds the kernel is the bytes a
+// compute unit takes in (128 KB a block at 16 heads of 128). 33 steps of 16
+// sequences through a layer of 72 heads of 64: 4.0 ms, 25.5 with a product
+// per head, as more heads than HG ran before, and 3.3 with 64 heads.
+constexpr int HG = 64; // heads whose values fit 64 KiB of LDS
 template <int NS>
 __global__ __launch_bounds__(1024) void heads_step_k(Heads d)
 {
-	extern __shared__ float red[]; // [nh][16 rows][16 channels]
+	extern __shared__ float red[]; // [min(nh, HG)][16 rows][16 channels]
 	const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), W = blockDim.x >> 6;
 	const int tc = (d.a.D + 15) / 16, r0 = (int)(blockIdx.x / (unsigned)tc) * 16, c0 = (int)(blockIdx.x % (unsigned)tc) * 16;
 	const int r = lane & 15, g = lane >> 4, nkb = d.Kp / 32;
-	for (int h = wave; h < d.a.nh; h += W) {
-		const long line0 = (long)h * d.a.rp + r0, ch0 = (long)h * d.a.Dp + c0;
-		const int8_t *A = d.q.dig + (line0 >> 5) * nkb * 3072 + ((line0 & 31) + r) * 16 + (g & 1) * 512 + (g >> 1) * 3072;
-		const int8_t *B = d.w + (ch0 >> 5) * nkb * 1024 + (g >> 1) * 1024 + ((g & 1) * 32 + (ch0 & 31) + r) * 16;
-		v4i af[NS][3], bf[NS];
+	const int t = threadIdx.x;
+	float s = 0.0f; // of threads 0 .. 255: their output's sum so far
+	for (int h0 = 0; h0 < d.a.nh; h0 += HG) {
+		const int hn = d.a.nh - h0 < HG ? d.a.nh - h0 : HG;
+		if (h0) __syncthreads(); // the values before are added
+		for (int h = h0 + wave; h < h0 + hn; h += W) {
+			const long line0 = (long)h * d.a.rp + r0, ch0 = (long)h * d.a.Dp + c0;
+			const int8_t *A = d.q.dig + (line0 >> 5) * nkb * 3072 + ((line0 & 31) + r) * 16 + (g & 1) * 512 + (g >> 1) * 3072;
+			const int8_t *B = d.w + (ch0 >> 5) * nkb * 1024 + (g >> 1) * 1024 + ((g & 1) * 32 + (ch0 & 31) + r) * 16;
+			v4i af[NS][3], bf[NS];
 #pragma unroll
-		for (int i = 0; i < NS; i++) {
-			bf[i] = *(const v4i *)(B + i * 2048);
+			for (int i = 0; i < NS; i++) {
+				bf[i] = *(const v4i *)(B + i * 2048);
 #pragma unroll
-			for (int l = 0; l < 3; l++) af[i][l] = *(const v4i *)(A + i * 6144 + l * 1024);
+				for (int l = 0; l < 3; l++) af[i][l] = *(const v4i *)(A + i * 6144 + l * 1024);
+			}
+			const int c = c0 + r;
+			const float sc = d.scale[ch0 + r];
+			int E[4], cls[4];
+#pragma unroll
+			for (int v = 0; v < 4; v++) E[v] = d.q.e[line0 + 4 * g + v], cls[v] = d.q.special[line0 + 4 * g + v];
+			v4i acc[3] = { { 0, 0, 0, 0 }, { 0, 0, 0, 0 }, { 0, 0, 0, 0 } };
+#pragma unroll
+			for (int i = 0; i < NS; i++)
+#pragma unroll
+				for (int l = 0; l < 3; l++) acc[l] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[i][l], bf[i], acc[l], 0, 0, 0);
+#pragma unroll
+			for (int v = 0; v < 4; v++) {
+				const int row = r0 + 4 * g + v;
+				const int cl = row < d.a.rows && c < d.a.D ? cls[v] : 0;
+				red[(h - h0) * 256 + (4 * g + v) * 16 + r] = sc * (cl == TGQ_GRID ? head_sum64(acc[0][v], acc[1][v], acc[2][v], E[v]) : line_value(d, h, row, c, E[v], cl));
+			}
 		}
-		const int c = c0 + r;
-		const float sc = d.scale[ch0 + r];
-		int E[4], cls[4];
-#pragma unroll
-		for (int v = 0; v < 4; v++) E[v] = d.q.e[line0 + 4 * g + v], cls[v] = d.q.special[line0 + 4 * g + v];
-		v4i acc[3] = { { 0, 0, 0, 0 }, { 0, 0, 0, 0 }, { 0, 0, 0, 0 } };
-#pragma unroll
-		for (int i = 0; i < NS; i++)
-#pragma unroll
-			for (int l = 0; l < 3; l++) acc[l] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[i][l], bf[i], acc[l], 0, 0, 0);
-#pragma unroll
-		for (int v = 0; v < 4; v++) {
-			const int row = r0 + 4 * g + v;
-			const int cl = row < d.a.rows && c < d.a.D ? cls[v] : 0;
-			red[h * 256 + (4 * g + v) * 16 + r] = sc * (cl == TGQ_GRID ? head_sum64(acc[0][v], acc[1][v], acc[2][v], E[v]) : line_value(d, h, row, c, E[v], cl));
-		}
+		__syncthreads();
+		if (t >= 256) continue;
+		for (int h = 0; h < hn; h++) s = h0 + h ? s + red[h * 256 + t] : red[t];
 	}
-	__syncthreads();
-	const int t = threadIdx.x, row = r0 + (t >> 4), c = c0 + (t & 15);
-	if (t >= 256 || row >= d.a.rows || c >= d.a.D) return;
-	float s = red[t];
-	for (int h = 1; h < d.a.nh; h++) s = s + red[h * 256 + t];
-	d.a.o[(long)row * d.a.orow + c] = s;
+	const int row = r0 + (t >> 4), c = c0 + (t & 15);
+	if (t < 256 && row < d.a.rows && c < d.a.D) d.a.o[(long)row * d.a.orow + c] = s;
 }
 
 // A prompt's rows: a block of 8 waves takes 64 rows x 128 channels, a wave 32
@@ -260,7 +268,7 @@ void tgk_heads(hipStream_t st, const tgk_heads_args *a, void *scratch)
 	}
 	const unsigned grid = (unsigned)((a->rows + 15) / 16 * ((a->D + 15) / 16));
 	const int W = a->nh < 4 ? 4 : a->nh < 16 ? a->nh : 16;
-	const size_t lds = (size_t)a->nh * 1024;
+	const size_t lds = (size_t)(a->nh < HG ? a->nh : HG) * 1024;
 	switch (w->Kp / 64) {
 	case 1: heads_step_k<1><<<grid, W * 64, lds, st>>>(d); break;
 	case 2: heads_step_k<2><<<grid, W * 64, lds, st>>>(d); break;

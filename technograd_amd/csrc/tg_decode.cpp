@@ -190,7 +190,7 @@ bool gemm_pre(tg_hip_dec *d, int wi, const float *x, long xr, int ni, long xj, i
 }
 
 // whether all heads' output projections run as one product (tgk_heads)
-bool heads_fused(const tg_hip_dec *d) { return d->HD > TGK_REFLOOP_K && d->HD <= TGK_HEADS_MAX && d->NQ <= 64; }
+bool heads_fused(const tg_hip_dec *d) { return d->HD > TGK_REFLOOP_K && d->HD <= TGK_HEADS_MAX; }
 
 // the graph's rmsnorm-then-gain of token rows, fused with the update of h
 // before it (mode 1: h += add; mode 2: h += the heads' output projections in

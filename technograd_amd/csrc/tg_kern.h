@@ -228,7 +228,7 @@ void tgk_dec_silu_mul(hipStream_t s, const float *gu, long gus, float *out, int 
  * weights. w: int8 codes (whatever the model's width), channel h Dp + c for
  * (head h, channel c), Dp = D padded to 256 with zero codes. rp: the rows
  * padded to 32; the x of padding rows is read and dropped. scratch:
- * tgk_qgemm_scratch(nh rp, w->Kp) bytes. TGK_REFLOOP_K < HD <= TGK_HEADS_MAX, nh <= 64. */
+ * tgk_qgemm_scratch(nh rp, w->Kp) bytes. TGK_REFLOOP_K < HD <= TGK_HEADS_MAX. */
 #define TGK_HEADS_MAX 256
 typedef struct {
 	const float *x;

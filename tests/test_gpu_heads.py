@@ -20,6 +20,8 @@ def device():
 @pytest.mark.parametrize("seqs,T0,HD,NQ,D,bits", [
     (3, 9, 48, 2, 72, 4),      # one 64-input step, its last 16 padding
     (2, 5, 64, 17, 64, 8),     # more heads than waves
+    (3, 4, 48, 65, 40, 4),     # one head more than a step adds at a time
+    (2, 3, 64, 144, 32, 8),    # two such groups and a part
     (5, 7, 112, 4, 300, 4),    # channels off the 16- and 256-wide tiles
     (2, 3, 192, 2, 128, 4),    # three steps
     (3, 4, 256, 2, 96, 8),     # four

@@ -186,3 +186,22 @@ except RuntimeError as e:
     assert "out of memory" in str(e)
 assert make(1 << 40) == (full, launches)
 """)
+
+
+def test_a_steps_launches_do_not_grow_with_the_heads(run):
+    """All heads' output projections of a decoder step are one product,
+    however many heads there are."""
+    run("""
+counts = []
+for NQ in (8, 64, 72, 144):
+    prog = hip.Program(synth.qwen3_tgir("q", T=8, rope_len=8, L=1, D=32, NQ=NQ, NKV=NQ // 8, HD=48, FF=32, V=96), max_rows=1)
+    dec = hip.Decoder(prog, 2, 4, 8)
+    prompt = hip.DeviceBuffer(4 * 8)
+    n = fake.fake_launches()
+    dec.generate_device(prompt.ptr, 2, 4, 1, None, None)
+    m = fake.fake_launches()
+    dec.generate_device(prompt.ptr, 2, 4, 2, None, None)
+    counts.append((m - n, fake.fake_launches() - m))
+    dec.close()
+assert len(set(counts)) == 1, counts
+""")
