@@ -99,18 +99,18 @@ __global__ __launch_bounds__(256) void fx_mm_k(tgk_fx_mm d)
 }
 
 // products of two row values (attention): one output per thread
-__global__ __launch_bounds__(256) void fx_mmrow_k(int *o, long R, tgk_fx a, tgk_fx b, int M, int K, int N, int rows)
+__global__ __launch_bounds__(256) void fx_mmrow_k(int *o, long R, tgk_fx a, tgk_fx b, int G, int M, int K, int N, int rows)
 {
 	const int row = blockIdx.x * 256 + threadIdx.x;
 	if (row >= rows) return;
-	for (long e = blockIdx.y; e < (long)M * N; e += gridDim.y) {
-		const int g = blockIdx.z;
-		const long i = e / N, j = e - i * N, ai = ((long)g * M + i) * K, bj = (long)g * K * N + j;
-		long s = 0;
+	for (int g = blockIdx.z; g < G; g += gridDim.z)
+		for (long e = blockIdx.y; e < (long)M * N; e += gridDim.y) {
+			const long i = e / N, j = e - i * N, ai = ((long)g * M + i) * K, bj = (long)g * K * N + j;
+			long s = 0;
 #pragma unroll 4
-		for (int p = 0; p < K; p++) s += (long)at(a, ai + p, row) * at(b, bj + (long)p * N, row);
-		o[((long)g * M * N + e) * R + row] = sat((s + 32768) >> 16);
-	}
+			for (int p = 0; p < K; p++) s += (long)at(a, ai + p, row) * at(b, bj + (long)p * N, row);
+			o[((long)g * M * N + e) * R + row] = sat((s + 32768) >> 16);
+		}
 }
 
 __global__ __launch_bounds__(256) void fx_bin_k(int op, int *o, long R, tgk_fx a, int am, const int *amap, tgk_fx b, int bm, const int *bmap,
@@ -259,8 +259,8 @@ void tgk_fx_mul(hipStream_t s, const tgk_fx_mm *d)
 void tgk_fx_mulrow(hipStream_t s, int *o, long R, tgk_fx a, tgk_fx b, int G, int M, int K, int N, int rows)
 {
 	dim3 g = grid2(rows, (long)M * N);
-	g.z = (unsigned)G;
-	fx_mmrow_k<<<g, 256, 0, s>>>(o, R, a, b, M, K, N, rows);
+	g.z = (unsigned)(G < 65535 ? G : 65535);
+	fx_mmrow_k<<<g, 256, 0, s>>>(o, R, a, b, G, M, K, N, rows);
 }
 
 void tgk_fx_binary(hipStream_t s, int op, int *o, long R, tgk_fx a, int am, const int *amap, tgk_fx b, int bm, const int *bmap, int n, int rows)

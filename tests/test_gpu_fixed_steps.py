@@ -49,6 +49,14 @@ MODELS = {
                  "    (%7 (f32 3) (mul i %6))\n    (%8 (f32 3 270) (outer %7 %5))\n    (%9 (f32 90 4) (sub %3 %0))\n"
                  "    (%10 (f32 360) (reshape %9))\n    (%11 (f32 3 360) (outer i %10))\n    (%12 (f32 3 270) (gelu %8))\n"
                  "    (%13 (f32) (sum %11))\n    (%14 (f32 3 270) (add %12 %13))\n", "%14"),
+    # groups of row values by row values, ragged; a scan from the last step to the first
+    "groups": model([], "  (input a (f32 7 5 33))\n  (input b (f32 7 33 19))\n",
+                    "    (%0 (f32 7 5 19) (matmul a b))\n    (%1 (f32 7 19 5) (transpose %0))\n    (%2 (f32 7 5 5) (matmul %0 %1))\n"
+                    "    (%3 (f32 7 5 5) (softmax %2))\n    (%4 (f32 7 5 19) (matmul %3 %0))\n", "%4"),
+    "reverse": model([f32("h0", 40, seed=8), quant("W", 40, 40, 8, 1, 9)], "  (input x (f32 6 40))\n",
+                     "    (scan 6 reverse steps\n      (carry %0 (f32 40) h0)\n      (in %1 (f32 40) x)\n      (body\n"
+                     "        (%2 (f32 40) (matmul %0 W))\n        (%3 (f32 40) (add %2 %1))\n        (%4 (f32 40) (tanh %3))\n      )\n"
+                     "      (next %0 %4)\n      (emit %5 (f32 6 40) %3)\n    )\n    (%6 (f32 6 40) (softmax %5))\n", "%6"),
 }
 
 
@@ -76,3 +84,10 @@ def test_steps_equal_interpreter(name, rows):
 def test_scans_equal_interpreter(rows):
     print("case fixed scan", rows, flush=True)
     check(synth.ssm_tgir(d_model=16, d_inner=32, n_state=4, dt_rank=4, T=7, blocks=2, classes=3), rows)
+
+
+def test_more_groups_than_a_grid_holds():
+    print("case fixed groups", flush=True)
+    G = 65535 + 3
+    text = model([], "  (input a (f32 %d 2 3))\n  (input b (f32 %d 3 1))\n" % (G, G), "    (%%0 (f32 %d 2 1) (matmul a b))\n" % G, "%0")
+    check(text, 2)

@@ -205,3 +205,14 @@ for NQ in (8, 64, 72, 144):
     dec.close()
 assert len(set(counts)) == 1, counts
 """)
+
+
+def test_any_number_of_groups_is_launched(run):
+    """A Q16.16 batched product of more groups than a grid has in its third
+    dimension."""
+    run("""
+for G in (65535, 65536, 200000):
+    text = ("(tgir 1\\n  (model m)\\n  (input a (f32 %d 2 3))\\n  (input b (f32 %d 3 1))\\n  (block\\n    (%%0 (f32 %d 2 1) (matmul a b))\\n"
+            "  )\\n  (output %%0))\\n" % (G, G, G))
+    hip.Program(text, flags=hip.FIXED, max_rows=2).batch_fixed(np.ones((2, G * 9), np.int32))
+""")
