@@ -1,6 +1,7 @@
 """Q16.16 programs too large to compile, run an instruction at a time, against
 the row-program interpreter: the same integers, for every kind of instruction,
-weights on both sides, rows off the multiples of a wave."""
+weights on both sides, rows off the multiples of a wave. That these models do
+run so, and not both ways in the interpreter, is test_host_calls.py's."""
 import numpy as np
 import pytest
 
@@ -80,14 +81,17 @@ def test_steps_equal_interpreter(name, rows):
     check(MODELS[name], rows)
 
 
+SCAN = synth.ssm_tgir(d_model=16, d_inner=32, n_state=4, dt_rank=4, T=7, blocks=2, classes=3)
+G = 65535 + 3  # more groups than a grid has in its third dimension
+GROUPS = model([], "  (input a (f32 %d 2 3))\n  (input b (f32 %d 3 1))\n" % (G, G), "    (%%0 (f32 %d 2 1) (matmul a b))\n" % G, "%0")
+
+
 @pytest.mark.parametrize("rows", [3, 130])
 def test_scans_equal_interpreter(rows):
     print("case fixed scan", rows, flush=True)
-    check(synth.ssm_tgir(d_model=16, d_inner=32, n_state=4, dt_rank=4, T=7, blocks=2, classes=3), rows)
+    check(SCAN, rows)
 
 
 def test_more_groups_than_a_grid_holds():
     print("case fixed groups", flush=True)
-    G = 65535 + 3
-    text = model([], "  (input a (f32 %d 2 3))\n  (input b (f32 %d 3 1))\n" % (G, G), "    (%%0 (f32 %d 2 1) (matmul a b))\n" % G, "%0")
-    check(text, 2)
+    check(GROUPS, 2)

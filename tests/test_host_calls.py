@@ -216,3 +216,21 @@ for G in (65535, 65536, 200000):
             "  )\\n  (output %%0))\\n" % (G, G, G))
     hip.Program(text, flags=hip.FIXED, max_rows=2).batch_fixed(np.ones((2, G * 9), np.int32))
 """)
+
+
+def test_the_fixed_step_models_run_an_instruction_at_a_time(run):
+    """Every model of test_gpu_fixed_steps.py takes the executor that the file
+    tests, a launch or more per instruction; the interpreter it is compared
+    with launches once a pass."""
+    run("""
+sys.path.insert(0, os.path.join(%r, "tests"))
+import test_gpu_fixed_steps as F
+for name, text in sorted(F.MODELS.items()) + [("scan", F.SCAN), ("groups", F.GROUPS)]:
+    n = []
+    for flags in (hip.FIXED, hip.FIXED | hip.INTERP):
+        p = hip.Program(text, flags=flags, max_rows=64)
+        a = fake.fake_launches()
+        p.batch_fixed(np.ones((3, p.per), np.int32))
+        n.append(fake.fake_launches() - a)
+    assert n[0] >= 3 and n[1] == 1, (name, n)
+""" % ROOT)
