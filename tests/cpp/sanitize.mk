@@ -22,7 +22,7 @@ SRC      = technograd_amd/csrc
 SAN      = -fsanitize=address,undefined,float-cast-overflow -fno-sanitize-recover=all -fno-omit-frame-pointer
 CFLAGS_S = -std=gnu11 -O1 -g -fPIC -pthread -ffp-contract=off -Wall -Wno-unused-function -Iinclude -I$(SRC) $(SAN)
 HOST_C   = tgir_read tgir_write tg_quant tg_gptq tg_front
-HIP_OBJ  = tg_hip tg_decode tg_rpgen kern_layer kern_qgemm kern_rowprog kern_decode
+HIP_OBJ  = tg_hip tg_decode tg_rpgen kern_layer kern_qgemm kern_rowprog kern_fixed kern_heads kern_decode
 export ASAN_OPTIONS  = detect_leaks=1:abort_on_error=1
 export UBSAN_OPTIONS = print_stacktrace=1:halt_on_error=1
 

@@ -30,3 +30,16 @@ def test_host_parsers_fuzz_clean_under_sanitizers():
     for mode in ("tgir:", "front:", "gptq:", "rows:", "http:"):
         assert mode in r.stdout, r.stdout
     assert "runtime error" not in r.stderr and "ERROR: AddressSanitizer" not in r.stderr, r.stderr[-4000:]
+
+
+def test_sanitized_library_links_every_object():
+    """The instrumented library is linked from the same objects as the
+    ordinary one (an undefined kernel launcher would only show when it is
+    loaded)."""
+    def objects(*args):
+        r = subprocess.run(["make", "-n", "-B", *args], cwd=ROOT, capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, r.stderr
+        links = [line for line in r.stdout.splitlines() if " -shared " in line]
+        assert len(links) == 1, links
+        return sorted(os.path.basename(w) for w in links[0].split() if w.endswith(".o"))
+    assert objects("-f", "tests/cpp/sanitize.mk", "_san/lib/libtg_hip.so") == objects("-C", "technograd_amd", "lib/libtg_hip.so")
