@@ -852,6 +852,42 @@ __global__ __launch_bounds__(256) void qexact_k(QExact d, int tn)
 	}
 }
 
+// The same of few terms an output and channel, where a tile would be mostly
+// padding: a thread per output, neighbours along the contiguous side of the
+// output, a thread's operands for eight k loaded before the first is added.
+template <int BITS>
+__global__ __launch_bounds__(256) void qexact_few_k(QExact d, unsigned total)
+{
+	const unsigned t = blockIdx.x * 256 + threadIdx.x;
+	if (t >= total) return;
+	unsigned r, j, c; // batch row, inner row, channel
+	if (d.oc == 1) {
+		const unsigned m = t / (unsigned)d.C;
+		c = t - m * (unsigned)d.C, r = m / (unsigned)d.ni, j = m - r * (unsigned)d.ni;
+	} else {
+		const unsigned u = t / (unsigned)d.ni;
+		j = t - u * (unsigned)d.ni, r = u / (unsigned)d.C, c = u - r * (unsigned)d.C;
+	}
+	const float *x = d.x + r * d.xr + j * d.xj;
+	const long w = c * d.cc;
+	auto code = [&](int k) {
+		const long i = w + k * d.ck;
+		return (float)(BITS == 8 ? (int)(int8_t)d.codes[i] : (int)(int8_t)(uint8_t)(d.codes[i >> 1] << (i & 1 ? 0 : 4)) >> 4);
+	};
+	float acc = 0.0f;
+	constexpr int U = 8;
+	int k = 0;
+	for (; k + U <= d.K; k += U) {
+		float a[U], b[U];
+#pragma unroll
+		for (int q = 0; q < U; q++) a[q] = x[(k + q) * d.xk], b[q] = code(k + q);
+#pragma unroll
+		for (int q = 0; q < U; q++) acc = acc + b[q] * a[q];
+	}
+	for (; k < d.K; k++) acc = acc + code(k) * x[k * d.xk];
+	d.o[r * d.orr + j * d.oj + c * d.oc] = d.scale[c] * acc;
+}
+
 // the quantized products of tgk_matmul_exact (g == 1)
 static void launch_qexact(hipStream_t s, const tgk_mm *d, int rows)
 {
@@ -871,9 +907,20 @@ static void launch_qexact(hipStream_t s, const tgk_mm *d, int rows)
 	// unit's second block runs beside the first at R = 1 and 2 (22 and 49 us). So R = 2 from 256 of its tiles
 	// (333 rows x 1000 channels: 49 us against 57 at R = 1; 128 rows: 39 against 22), and R = 4, which does the
 	// most per LDS read, once its tiles fill the chip twice (4096 rows: 286 us against 390).
+	// A thread per output where a tile is mostly padding, measured over C = 1 .. 128, K = 2 .. 128 and 1000, 65536 and
+	// 10^6 activation rows. x @ W and W @ x with inner rows (neighbours read neighbouring codes, or one): to C K = 640
+	// (65536 rows, C = 16: K = 32 10 us against 16, K = 128 32 against 37; C = 64: K = 8 14 against 15, K = 16 20 against
+	// 18). W @ x of one vector a row (codes K apart): to 192, 32 channels and, past 8 channels, 12 inputs (10^6 rows, C =
+	// 1, K = 8: 18 us against 141; 65536, C = 16: K = 12 10 against 12, K = 16 18 against 13). Few outputs leave either
+	// form a launch's latency: short chains take less of it here (1000 rows x 128 channels, K = 8: 3.8 us against 4.9),
+	// long ones in a tile (1000 x 1, K = 24: 4.6 against 4.1, K = 64: 9 against 4).
+	const long total = M * e.C, CK = (long)e.C * e.K;
+	const bool apart = e.oc == 1 && e.cc != 1, pad = apart ? CK <= 192 && e.C <= 32 && (e.K <= 12 || e.C <= 8) : CK <= 640;
+	const bool few = total < (1L << 32) && (e.K <= 12 ? pad || total <= 131072 : pad && total >= 16384);
 	auto run = [&](auto bits) {
 		constexpr int B = decltype(bits)::value;
-		if (tiles(64) >= 512) qexact_k<4, B><<<(unsigned)tiles(64), 256, 0, s>>>(e, (e.C + 63) / 64);
+		if (few) qexact_few_k<B><<<blocks_for(total), 256, 0, s>>>(e, (unsigned)total);
+		else if (tiles(64) >= 512) qexact_k<4, B><<<(unsigned)tiles(64), 256, 0, s>>>(e, (e.C + 63) / 64);
 		else if (tiles(32) >= 256) qexact_k<2, B><<<(unsigned)tiles(32), 256, 0, s>>>(e, (e.C + 31) / 32);
 		else qexact_k<1, B><<<(unsigned)tiles(16), 256, 0, s>>>(e, (e.C + 15) / 16);
 	};

@@ -4,12 +4,14 @@ each tile's edges, both weight widths and both operand layouts."""
 import numpy as np
 import pytest
 
-from technograd_amd import hip
+from technograd_amd import hip, synth
 
 pytestmark = pytest.mark.gpu
 
 # rows, inputs, channels: the three tile sizes with partial rows, channels and last chunks
 SHAPES = [(1, 5, 3), (17, 129, 33), (15, 128, 16), (290, 67, 1021), (256, 64, 1024), (2049, 37, 1025)]
+# and a thread per output: fewer terms than are read ahead, as many, one more; a block's last threads
+SHAPES += [(1, 1, 1), (300, 7, 5), (129, 8, 2), (40001, 9, 1), (16385, 33, 4), (1031, 24, 127)]
 
 
 @pytest.fixture(scope="module", autouse=True)
@@ -26,7 +28,8 @@ def pack(codes, bits):
     return ((c[0::2] & 15) | ((c[1::2] & 15) << 4)).astype(np.uint8).view(np.int8)
 
 
-@pytest.mark.parametrize("axis", [0, 1])
+# W @ X, X @ W, and W @ x for a vector x per row
+@pytest.mark.parametrize("axis", [0, 1, "vector"])
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("shape", SHAPES)
 def test_sequential_sums(shape, bits, axis):
@@ -44,7 +47,11 @@ def test_sequential_sums(shape, bits, axis):
         for k in range(K):  # the reference's loop: a rounded product, then a rounded add
             want = want + x[:, k, None] * codes[None, :, k].astype(np.float32)
         want = want * scales
-    if axis == 1:
+    if axis == "vector":
+        text = "(tgir 1\n  (model m)\n%s  (input x (f32 %d))\n  (block\n    (%%0 (f32 %d) (matmul W x))\n  )\n  (output %%0))\n" % (
+            synth.param_quant("W", codes, scales, bits, 0), K, C)
+        got = hip.Program(text, flags=hip.EXACT, max_rows=M).batch(x)[0]
+    elif axis == 1:
         got = hip.matmul_q(pack(np.ascontiguousarray(codes.T), bits), bits, scales, x, M, K, C, 1, flags=hip.EXACT)
     else:
         got = hip.matmul_q(pack(codes, bits), bits, scales, np.ascontiguousarray(x.T), C, K, M, 0, flags=hip.EXACT).T
