@@ -295,10 +295,12 @@ __global__ void rowop_k(int op, float *o, long ors, tgk_opd a, int nrow, int col
 }
 
 // The same per-line results with the lines staged through LDS: a block takes
-// up to lpb consecutive lines of one batch row (its last block what is left),
-// which are contiguous in memory, so loads and stores are coalesced. Only the sums
-// keep one thread per line, walking its line in the reference's order; the
-// max, the exponentials, the division and the rmsnorm scaling are
+// lpb consecutive lines of the pass (the last block what is left), line L the
+// line L % nrow of batch row L / nrow. Within a batch row lines are contiguous
+// in memory, so loads and stores are coalesced; FLAT: so are all of them (rows
+// back to back on both sides), else each line's offsets are kept next to it.
+// Only the sums keep one thread per line, walking its line in the reference's
+// order; the max, the exponentials, the division and the rmsnorm scaling are
 // elementwise or order-free and use every thread. LDS lines are `stride`
 // floats apart, stride odd, so the sequential walks fall in distinct banks.
 // Softmax's max: x[0] when it is nan, else the largest of x[0] and the
@@ -315,13 +317,23 @@ __device__ inline float line_sum(const float *z, int cols)
 	return sum;
 }
 
-__global__ __launch_bounds__(256) void rowop_lds_k(int op, float *o, long ors, tgk_opd a, int nrow, int cols, int lpb, int stride)
+constexpr int ROWOP_LPB = 32; // lines a block takes at most
+template <bool FLAT>
+__global__ __launch_bounds__(256) void rowop_lds_k(int op, float *o, long ors, tgk_opd a, int nrow, long lines, int cols, int lpb, int stride)
 {
 	extern __shared__ float lds[];
+	__shared__ long in_off[ROWOP_LPB], out_off[ROWOP_LPB]; // !FLAT
 	float *lv = lds + lpb * stride; // one value per line (max, then sum or inverse rms)
-	const int bpr = (nrow + lpb - 1) / lpb, r = blockIdx.x / bpr, q0 = (blockIdx.x - r * bpr) * lpb;
-	const int nl = nrow - q0 < lpb ? nrow - q0 : lpb, tot = nl * cols; // (lines past nl: nothing is loaded, summed or stored)
-	const float *x = a.p + (long)r * a.rs + (long)q0 * cols;
+	const long L0 = (long)blockIdx.x * lpb;
+	const int nl = lines - L0 < lpb ? (int)(lines - L0) : lpb, tot = nl * cols; // (lines past nl: nothing is loaded, summed or stored)
+	const float *x = a.p + L0 * cols;
+	if (!FLAT) {
+		if ((int)threadIdx.x < nl) {
+			const long L = L0 + threadIdx.x, r = L / nrow, q = L - r * nrow;
+			in_off[threadIdx.x] = r * a.rs + q * cols, out_off[threadIdx.x] = r * ors + q * cols;
+		}
+		__syncthreads();
+	}
 	// element e of the tile is line e / cols, column e % cols: a thread's
 	// elements e, e + TPB, ... are walked by adding TPB as (dl lines, dc
 	// columns), with one carry, instead of a division per element
@@ -332,12 +344,13 @@ __global__ __launch_bounds__(256) void rowop_lds_k(int op, float *o, long ors, t
 	};
 	constexpr int U = 8;
 	{
-		int l = l0, c = c0;
+		int l = l0, c = c0, ll = l0, lc = c0;
 		for (int e0 = 0; e0 < tot; e0 += U * TPB) {
 			float v[U];
 			for (int j = 0; j < U; j++) {
 				const int e = e0 + j * TPB + threadIdx.x;
-				v[j] = x[e < tot ? e : tot - 1];
+				if (FLAT) v[j] = x[e < tot ? e : tot - 1];
+				else v[j] = a.p[in_off[e < tot ? ll : 0] + (e < tot ? lc : 0)], step(ll, lc);
 			}
 			for (int j = 0; j < U; j++) {
 				const int e = e0 + j * TPB + threadIdx.x;
@@ -377,8 +390,7 @@ __global__ __launch_bounds__(256) void rowop_lds_k(int op, float *o, long ors, t
 		}
 	}
 	__syncthreads();
-	float *out = o + (long)r * ors + (long)q0 * cols;
-	for (int e = threadIdx.x, ll = l0, c = c0; e < tot; e += TPB, step(ll, c)) out[e] = lds[ll * stride + c];
+	for (int e = threadIdx.x, ll = l0, c = c0; e < tot; e += TPB, step(ll, c)) o[FLAT ? L0 * cols + e : out_off[ll] + c] = lds[ll * stride + c];
 }
 
 // sum / mean of each row, one thread per row adding in index order (the
@@ -945,27 +957,26 @@ void tgk_matmul_exact(hipStream_t s, const tgk_mm *d, int rows)
 
 void tgk_rowop(hipStream_t s, int op, float *o, long ors, tgk_opd a, int nrow, int cols, int rows)
 {
-	long total = (long)rows * nrow;
+	const long total = (long)rows * nrow;
 	if (total <= 0) return;
-	if (a.rs == (long)nrow * cols && ors == (long)nrow * cols && total < (1L << 31)) {
-		// rows back to back in memory on both sides: all lines of the pass are one row's lines
-		// (lets one-line rows, such as one token each, share blocks)
-		nrow = (int)total;
-		rows = 1;
-	}
+	const bool flat = a.rs == (long)nrow * cols && ors == (long)nrow * cols; // rows back to back in memory on both sides
 	// lines 16-byte aligned and 4 banks apart when cols is a multiple of 4, else an odd stride
 	const int stride = cols % 4 == 0 ? cols + 4 : cols | 1;
 	// LDS: the lines and one value per line (padded to 4)
 	auto lds_bytes = [&](long l) { return (l * stride + ((l + 3) & ~3L)) * 4; };
-	// a power of two, so TPB / lpb threads of one wave share a line's max; few lines: spread over more blocks. Any number
-	// of lines takes this kernel: 1750 lines of 512 (not a multiple of four) ran one thread a line, 226 us against 11
-	int lpb = 32;
-	while (lpb > 4 && (lds_bytes(lpb) > 65536 || (long)rows * ((nrow + lpb - 1) / lpb) < 512)) lpb >>= 1;
-	const long grid = (long)rows * ((nrow + lpb - 1) / lpb);
-	if (cols >= 32 && lds_bytes(lpb) <= 65536 && grid < (1L << 31))
-		rowop_lds_k<<<(unsigned)grid, TPB, (size_t)lds_bytes(lpb), s>>>(op, o, ors, a, nrow, cols, lpb, stride);
-	else
+	auto grid = [&](int l) { return (total + l - 1) / l; };
+	// Lines per block: a power of two, so TPB / lpb threads of one wave share a line's max, and as many as leave 512
+	// blocks. Where the blocks do not all fit at once, no more than 17 KB of them, so that eight are on a unit and one's
+	// sums overlap another's loads (65536 lines of 512: 66 us at 8 a block, 69 at 16, 85 at 4; 30000 of 1000: 76 at 4,
+	// 105 at 8); where they do, more lines a block (8192 of 1024: 27 us at 8 a block, 34 at 4).
+	int lpb = ROWOP_LPB;
+	while (lpb > 4 && (lds_bytes(lpb) > 65536 || grid(lpb) < 512 || (lds_bytes(lpb) > 17500 && grid(lpb) > 256 * (163840 / lds_bytes(lpb))))) lpb >>= 1;
+	if (cols >= 32 && lds_bytes(lpb) <= 65536 && grid(lpb) < (1L << 31)) {
+		if (flat) rowop_lds_k<true><<<(unsigned)grid(lpb), TPB, (size_t)lds_bytes(lpb), s>>>(op, o, ors, a, nrow, total, cols, lpb, stride);
+		else rowop_lds_k<false><<<(unsigned)grid(lpb), TPB, (size_t)lds_bytes(lpb), s>>>(op, o, ors, a, nrow, total, cols, lpb, stride);
+	} else {
 		rowop_k<<<blocks_for(total), TPB, 0, s>>>(op, o, ors, a, nrow, cols, total);
+	}
 }
 
 namespace {
