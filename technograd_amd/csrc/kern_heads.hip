@@ -248,12 +248,12 @@ __global__ __launch_bounds__(512, 4) void heads_prompt_k(Heads d)
 
 } // namespace
 
-void tgk_heads(hipStream_t st, const tgk_heads_args *a, void *scratch)
+bool tgk_heads(hipStream_t st, const tgk_heads_args *a, void *scratch)
 {
 	const tgk_qweight *w = a->w;
 	if (!w || w->bits != 8 || a->rows <= 0 || a->nh <= 0 || a->HD <= TGK_REFLOOP_K || a->HD > TGK_HEADS_MAX || a->rp % 32 || a->rp < a->rows ||
 	    a->Dp % 256)
-		return;
+		return false;
 	tgk_qgemm_args g;
 	memset(&g, 0, sizeof g);
 	g.w = w, g.x = a->x, g.xr = a->xhead, g.xj = a->xrow, g.xk = 1, g.ni = a->rp, g.M = a->nh * a->rp;
@@ -264,7 +264,7 @@ void tgk_heads(hipStream_t st, const tgk_heads_args *a, void *scratch)
 		const unsigned grid = (unsigned)((a->rows + 63) / 64 * (a->Dp / 128));
 		if (w->Kp % 128 == 0) heads_prompt_k<4><<<grid, 512, 0, st>>>(d);
 		else heads_prompt_k<2><<<grid, 512, 0, st>>>(d);
-		return;
+		return true;
 	}
 	const unsigned grid = (unsigned)((a->rows + 15) / 16 * ((a->D + 15) / 16));
 	const int W = a->nh < 4 ? 4 : a->nh < 16 ? a->nh : 16;
@@ -275,4 +275,5 @@ void tgk_heads(hipStream_t st, const tgk_heads_args *a, void *scratch)
 	case 3: heads_step_k<3><<<grid, W * 64, lds, st>>>(d); break;
 	default: heads_step_k<4><<<grid, W * 64, lds, st>>>(d); break;
 	}
+	return true;
 }

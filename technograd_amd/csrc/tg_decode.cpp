@@ -272,7 +272,7 @@ bool forward(tg_hip_dec *d, int S, int T0, int p0)
 			ha.x = d->att, ha.xrow = (long)d->NQ * d->HD, ha.xhead = d->HD, ha.rows = rows, ha.rp = rp, ha.digits = head_digits;
 			ha.nh = d->NQ, ha.HD = d->HD, ha.D = d->D, ha.Dp = (d->D + 255) / 256 * 256;
 			ha.w = &d->ws[(size_t)d->wo[(size_t)l]], ha.o = d->dbuf, ha.orow = D;
-			tgk_heads(st, &ha, d->scratch);
+			if (!tgk_heads(st, &ha, d->scratch)) return err("decoder: output projections outside the kernel's sizes");
 			res = norm(d, 1, d->h, D, rows, d->dbuf, D, d->ln2[(size_t)l], d->n, d->wgu[(size_t)l]);
 		} else {
 			for (int hh = 0; hh < d->NQ; hh++)

@@ -228,7 +228,8 @@ void tgk_dec_silu_mul(hipStream_t s, const float *gu, long gus, float *out, int 
  * weights. w: int8 codes (whatever the model's width), channel h Dp + c for
  * (head h, channel c), Dp = D padded to 256 with zero codes. rp: the rows
  * padded to 32; the x of padding rows is read and dropped. scratch:
- * tgk_qgemm_scratch(nh rp, w->Kp) bytes. TGK_REFLOOP_K < HD <= TGK_HEADS_MAX. */
+ * tgk_qgemm_scratch(nh rp, w->Kp) bytes. TGK_REFLOOP_K < HD <= TGK_HEADS_MAX. False, with nothing launched,
+ * for sizes outside this. */
 #define TGK_HEADS_MAX 256
 typedef struct {
 	const float *x;
@@ -239,7 +240,7 @@ typedef struct {
 	long orow;
 	int digits; /* the scratch holds the lines' digits already (line head rp + row; those of padding rows may be anything) */
 } tgk_heads_args;
-void tgk_heads(hipStream_t s, const tgk_heads_args *a, void *scratch);
+bool tgk_heads(hipStream_t s, const tgk_heads_args *a, void *scratch);
 /* causal softmax over a prompt chunk's scores sc [lines][T0] (line L is
  * position L % T0 of its sequence and head): x = s * scale + 0 and the
  * softmax on u <= t, p = 0 above the diagonal, up to the end of the line's
