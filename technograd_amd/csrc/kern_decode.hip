@@ -592,8 +592,9 @@ template <int LPL, int QPL, int NL> void norm_lines(hipStream_t s, const NormLin
 	else norm_lines_k<LPL, QPL, NL, false><<<grid, 256, lds, s>>>(n);
 }
 
-// whether lines padded to Kp run there, and the launch
-// (4096: a block holds one line either way, and dec_norm_k is that kernel)
+// whether lines padded to Kp run there, and the launch (4096: a line's quads
+// are a block's registers; dec_norm_k, a line a block, takes 320 us for 4096
+// rows of 4096 and 1.27 ms for 16384)
 bool norm_lines_for(hipStream_t s, int Kp, const NormLines &n)
 {
 	switch (Kp) {

@@ -53,9 +53,11 @@ typedef const int __attribute__((address_space(4))) *cword;
 // wave: they come through scalar loads, CH words at a time from the packed
 // copy [C/16][K][16], and a term is one v_mad_i64_i32 with a scalar operand.
 // Four waves of a block take neighbouring channels of the same 64 rows. It is
-// bound by those multiply-adds (about 11 cycles each on a SIMD). 16384 rows x
-// 256 inputs x 256 channels take about 75 us, a 64-256-256-16 MLP's pass of
-// those rows 138 us; the interpreter took 12.5 ms for it.
+// bound by VALU issue and, for the rest, by loads: at 16384 rows, 64 inputs to
+// 256 channels and 256 to 256, a SIMD issues an instruction (four cycles,
+// v_mad_i64_i32 too) in 70 % of its cycles, and its four waves wait 41 % of
+// theirs. 16384 rows x 256 inputs x 256 channels take 65 us, a 64-256-256-16
+// MLP's pass of those rows 138 us; the interpreter took 12.5 ms for it.
 template <int CH>
 __global__ __launch_bounds__(256) void fx_mm_k(tgk_fx_mm d)
 {

@@ -25,7 +25,7 @@ def test_widths_equal_fixed_length_forward(D, FF, HD):
 
 # prompts of 2048 token rows and more: the many-lines norms, at every padded width, ragged and whole, lines off a block's
 @pytest.mark.parametrize("seqs,T0,D,HD", [(33, 63, 64, 64), (33, 63, 100, 128), (41, 50, 256, 48), (33, 63, 509, 256), (33, 63, 1024, 32),
-                                          (16, 128, 2047, 64), (16, 129, 2112, 16)])
+                                          (16, 128, 2047, 64), (16, 129, 2112, 16), (16, 128, 2048, 64), (21, 100, 4040, 48), (16, 128, 4096, 16)])
 def test_many_lines_equal_fixed_length_forward(seqs, T0, D, HD):
     print("case many lines", seqs, T0, D, HD, flush=True)
     check_decode(seqs, T0, 2, dict(L=2, D=D, NQ=2, NKV=1, HD=HD, FF=64, V=96))
