@@ -2607,7 +2607,7 @@ bool host_pipe_init(tg_hip_prog *p)
 }
 
 // Host buffers, the block loop of `tgc batch`: rows go in chunks through a
-// pipeline of NSL slots. Chunk i uses slot i % NSL: its rows are copied into
+// pipeline of slots. Chunk i uses slot i % nsl: its rows are copied into
 // the slot's pinned buffer on the host, up to the device on the copy-in
 // stream, computed on the program's stream, and down on the copy-out stream;
 // each stream waits for the event of the step before it. A chunk whose
@@ -2620,6 +2620,10 @@ bool host_pipe_init(tg_hip_prog *p)
 // events between three. 8192 rows of 512 values in and out, pageable, through a
 // 512-2048-2048-512 MLP: 1.41-1.51 ms in one chunk and three slots,
 // 0.9-1.1 now; 3000 rows 0.91 ms down three streams, 0.56 down one.
+// Three slots where rows or outputs travel directly: transfers that no host
+// copy paces queue up, and with a fourth chunk's ahead they no longer go both
+// ways at once (65536 rows of 512 values through a 512-512-512 MLP, both
+// direct: 3.5 ms, 5.2 with four slots; rows or outputs staged 3.4 and 4.0).
 int batch_host(tg_hip_prog *p, const void *rows, long nrows, void *out, int *steps)
 {
 	if (!p) {
@@ -2636,6 +2640,7 @@ int batch_host(tg_hip_prog *p, const void *rows, long nrows, void *out, int *ste
 	// stages, so that what nothing overlaps (the first one's way in, the last one's way out) is short
 	const long cmax = din && dout ? std::min(h.chunk, std::max(64L, (h.chunk + 1) / 2)) : h.chunk;
 	const long nch0 = (nrows + cmax - 1) / cmax, C = nch0 > 1 ? (nrows + nch0 - 1) / nch0 : cmax, nch = (nrows + C - 1) / C;
+	const int nsl = din || dout ? 3 : NSL;
 	const hipStream_t up = nch > 1 ? h.h2d : p->st, down = nch > 1 ? h.d2h : p->st;
 	float ms_total = 0;
 	// Pieces of each slot's copies; neither they nor anything queued on the device outlives the call, whatever it
@@ -2659,7 +2664,7 @@ int batch_host(tg_hip_prog *p, const void *rows, long nrows, void *out, int *ste
 	long arrived = 0; // chunks before it are down, their copies to the caller begun
 	auto arrive = [&](bool wait) -> bool { // the next chunk's outputs, if they are down (or once they are)
 		const long i = arrived, r0 = i * C, cnt = nrows - r0 < C ? nrows - r0 : C;
-		const int k = (int)(i % NSL);
+		const int k = (int)(i % nsl);
 		const hipError_t e = wait ? hipEventSynchronize(h.down[k]) : hipEventQuery(h.down[k]);
 		if (e == hipErrorNotReady) {
 			(void)hipGetLastError(); // an answer, not an error: the next pass's launch check must not find it
@@ -2675,10 +2680,10 @@ int batch_host(tg_hip_prog *p, const void *rows, long nrows, void *out, int *ste
 		return true;
 	};
 	for (long i = 0; i < nch; i++) {
-		const int k = (int)(i % NSL);
+		const int k = (int)(i % nsl);
 		const long r0 = i * C, cnt = nrows - r0 < C ? nrows - r0 : C;
-		if (i >= NSL) { // the slot's previous chunk is out: its buffers are free
-			if (arrived <= i - NSL && !arrive(true)) return -1;
+		if (i >= nsl) { // the slot's previous chunk is out: its buffers are free
+			if (arrived <= i - nsl && !arrive(true)) return -1;
 			p->copies->wait(left.out[k]);
 		}
 		const void *src = (const char *)rows + (size_t)r0 * per * 4;

@@ -60,15 +60,16 @@ for n in (8, 29, 200):
 """)
 @pytest.mark.parametrize("max_rows", [1, 7, 33, 63, 64, 65, 300])
 def test_pinned_rows_stay_in_the_slots(run, max_rows):
-    """Rows and outputs that are both pinned travel in chunks no larger than
-    the slots, which hold at most max_rows rows."""
+    """Rows and outputs, pinned or not, travel in chunks no larger than the
+    slots, which hold at most max_rows rows."""
     run("""
 prog = hip.Program(linear(64, 40), max_rows=%d)
 for n in (1, 2, 32, 63, 64, 65, 129, 500):
     (bx, x), (by, y) = pinned(np.ones((n, 64), np.float32)), pinned(np.zeros((n, 40), np.float32))
-    prog.batch(x, y)
-    assert fake.fake_out_of_range() == 0, n
-    assert fake.fake_pending() == 0, n
+    for rows, out in ((x, y), (x, np.array(y)), (np.array(x), y), (np.array(x), np.array(y))):
+        prog.batch(rows, out)
+        assert fake.fake_out_of_range() == 0, n
+        assert fake.fake_pending() == 0, n
     bx.free(), by.free()
 """ % max_rows)
 
