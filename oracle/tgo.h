@@ -9,7 +9,7 @@
  * (src/main.c:400-444, src/par.c).
  *
  * Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may
- * load this library, and only as the checker. The product (technograd_amd/)
+ * load this library, and only to compare with. The product (technograd_amd/)
  * never links it.
  *
  * Parity status per function is recorded in the header comment of each
